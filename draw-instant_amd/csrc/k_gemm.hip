@@ -1,6 +1,7 @@
 // Host side of the MFMA GEMM / implicit-GEMM conv (k_gemm_kernel.h): plan
 // selection, the split-K reducers and launch_gemm, which dispatches to the
 // instantiation families of k_gemm_*.hip.
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -616,6 +617,48 @@ static void env_plan_override(const GemmArgs& g, int elem, const char* env_tile,
   if (plan->splits < 1) plan->splits = 1;
 }
 
+// Plan of a split-operand fp32 problem (k_gemm_f32.hip) from what its tiles
+// measure on a MI355X: microseconds per 32-deep stage of one workgroup that
+// has its CU to itself (`alone`: barriers and LDS round trips in series) and
+// of each of the `res` workgroups that a CU holds (`shared`: 165-180 TFLOP/s
+// whole chip).  A stage of all rounds costs a CU the full rounds' shared time
+// plus the last round's, which falls no lower than one workgroup's own; a
+// split adds a reducer (3 us and its traffic at 3.5 TB/s).  The model's
+// choices are within 6 % of the best of a timed sweep of every tile and 1-64
+// splits over nineteen shapes (1 x 1280 x 1280 to 2048 x 5120 x 1280 linears,
+// 256 x 64 x 256 to 2304 x 2304 x 64 batches, 4 -> 320 to 1280 -> 1280
+// convolutions at 8 x 8 to 72 x 72).
+static GemmPlan f32_plan(const GemmArgs& g, int num_cus) {
+  struct Tile {
+    int id;
+    uint32_t bm, bn, res;
+    double alone, shared;
+  };
+  static const Tile tiles[] = {{TILE_128x128, 128, 128, 2, 1.7, 1.35},
+                               {TILE_128x64, 128, 64, 3, 1.2, 0.76},
+                               {TILE_64x64, 64, 64, 4, 0.88, 0.45}};
+  const uint32_t stages = (g.K + 31) / 32;
+  GemmPlan best{TILE_64x64, 1};
+  double best_t = 1e300;
+  for (const Tile& t : tiles) {
+    const uint64_t T = (uint64_t)((g.M + t.bm - 1) / t.bm) * ((g.N + t.bn - 1) / t.bn) * g.batch;
+    for (uint32_t s = 1; s <= 64 && s <= stages; s++) {
+      const uint32_t per = (stages + s - 1) / s;
+      if (s > 1 && (per < 2 || (stages + per - 1) / per != s || T * s > 65535ull * 64)) continue;
+      const uint64_t w = (T * s + num_cus - 1) / num_cus;  // workgroups of the fullest CU
+      const uint64_t rem = w % t.res;
+      double us = (double)per * ((double)(w - rem) * t.shared +
+                                 (rem ? std::max(t.alone, rem * t.shared) : 0.0));
+      if (s > 1) us += 3.0 + (double)g.batch * g.M * g.N * 4.0 * (s + 1) / 3.5e6;
+      if (us < best_t) {
+        best_t = us;
+        best = GemmPlan{t.id, s};
+      }
+    }
+  }
+  return best;
+}
+
 GemmPlan gemm_plan(const GemmArgs& g, int elem, int num_cus) {
   // DI_GEMM_PLAN="M,N,K,tile,splits;..." fixes the plan of the listed fp16
   // shapes only (tuning runs of the whole step; tile 13 = the halo conv)
@@ -657,8 +700,8 @@ GemmPlan gemm_plan(const GemmArgs& g, int elem, int num_cus) {
     return best;
   }
   if (elem == DI_F32) {
-    uint64_t t = (uint64_t)((g.M + 127) / 128) * ((g.N + 127) / 128) * g.batch;
-    best.tile = t >= (uint64_t)num_cus / 2 ? TILE_128x128 : TILE_64x64;
+    best = f32_plan(g, num_cus);  // (the bounds-checked fp32 kernel: any split of it, one tile)
+    env_plan_override(g, elem, env_tile, env_split, &best);
     return best;
   }
   const double cus = num_cus;
@@ -841,6 +884,9 @@ void launch_gemm(GemmArgs g, int elem, int a_mode, int b_mode, int tile_cfg, hip
     else if (a_mode == A_DENSE && g.rstats) gemm_fast_dense_ex(g, tile_cfg, s);
     else if (a_mode == A_DENSE) gemm_fast_dense(g, tile_cfg, s);
     else gemm_fast_conv(g, tile_cfg, s);
+  } else if (elem == DI_F32 && gemm_f32_ok(g, a_mode, b_mode)) {
+    gemm_f32(g, a_mode, b_mode, tile_cfg, s);  // with its own split-K reducer
+    return;
   } else {
     gemm_slow(g, elem, a_mode, b_mode, tile_cfg, s);
   }

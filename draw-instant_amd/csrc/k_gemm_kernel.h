@@ -12,7 +12,8 @@
 //    (Upsample2D), and a channel concat of two sources (up-block skips);
 //  * the reference's fp32 ops (matmul wgsl-ops.js:477-556, gemm :821-897,
 //    convMM :584-698 with its (ci, ky, kx) k order on NCHW) through an fp32
-//    MFMA variant with exact fp32 products.
+//    MFMA variant with exact fp32 products, where an operand is too large for
+//    k_gemm_f32.hip.
 // Epilogue: alpha, per-column bias, per-(batch, column) bias (ResNet temb),
 // residual add, GELU(erf) / GEGLU / SiLU, fp16 or fp32 store, NHWC or NCHW.
 //
@@ -1200,10 +1201,14 @@ void launch_cfg(const GemmArgs& g, hipStream_t s) {
       <<<dim3(tiles, 1, g.batch * g.splits), 64 * WGM * WGN * KS, 0, s>>>(g);
 }
 
-// Generic (bounds-checked) variants: two tile shapes.
+// Generic (bounds-checked) variants: two tile shapes, one for fp32 (operands
+// past the split kernel's 31-bit offsets).
 template <typename T, int AM, int BMD, typename TB = T>
 void launch_slow(const GemmArgs& g, int tile_cfg, hipStream_t s) {
-  if (tile_cfg == TILE_64x64 || tile_cfg == TILE_128x64 || tile_cfg == TILE_64x128 ||
+  if constexpr (sizeof(T) == 4) {
+    launch_cfg<T, 64, 64, 2, 2, AM, BMD, false, 2, 1, EX_NONE, TB>(g, s);
+    return;
+  } else if (tile_cfg == TILE_64x64 || tile_cfg == TILE_128x64 || tile_cfg == TILE_64x128 ||
       tile_cfg == TILE_64x160 || tile_cfg == TILE_64x64_K2 || tile_cfg == TILE_128x64_K2 ||
       tile_cfg == TILE_64x128_K2 || tile_cfg == TILE_64x128_W16 || tile_cfg == TILE_128x64_W16 ||
       tile_cfg == TILE_64x64_W16)

@@ -16,7 +16,13 @@ int run_gemm(di_ctx* ctx, GemmArgs& g, int elem, int a_mode, int b_mode, int til
   if (g.splits > 1) {
     void* ws = nullptr;
     int rc = workspace(ctx, gemm_ws_bytes(g), &ws);
-    if (rc) return rc;
+    if (rc && elem == DI_F32) {
+      // no memory for the partials: fp32 problems also run in one piece
+      (void)hipGetLastError();
+      g.splits = 1;
+    } else if (rc) {
+      return rc;
+    }
     g.part = (float*)ws;
   }
   launch_gemm(g, elem, a_mode, b_mode, tile, ctx->stream);

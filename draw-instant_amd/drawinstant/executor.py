@@ -1806,7 +1806,7 @@ class Executor:
                  conv_f16: bool = False):
         """``conv_f16`` (opt-in): Conv nodes run on the fp16 MFMA path
         (DI_CONV_F16_COMPUTE: fp32 tensors staged to fp16 operands, fp32
-        accumulation and output) instead of the exact fp32 MFMA path the
+        accumulation and output) instead of the fp32 path the
         reference's fp32 semantics call for."""
         self.device = device
         self.graph = graph

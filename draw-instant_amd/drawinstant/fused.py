@@ -162,7 +162,7 @@ def run_conv_bench(device: Optional[Device] = None, shape=None, on_progress=None
                    return_tensors: bool = False):
     """conv3x3 with the WGSL_CONV epilogue silu(conv + bias) + residual.
     naive: conv -> SiLU -> Add (3 dispatches); fused: one di_conv2d with
-    DI_CONV_SILU and the residual.  fp32 NCHW, exact fp32 MFMA.
+    DI_CONV_SILU and the residual.  fp32 NCHW.
 
     ``return_tensors`` adds ``tensors``: the host inputs (x, w, bias, r in
     NCHW / OIHW) and the fused output y, for a parity check of the fused
@@ -445,7 +445,7 @@ def run_block_bench(device: Optional[Device] = None, shape=None, on_progress=Non
     return bn.finish(S, naive, fused, lambda: bn.read(yn, (nrd,)), lambda: bn.read(yf, (nrd,)),
                      11 + nd_attn, 9, repeats, warm_ms,
                      flops=2.0 * rows * D * D * 4 + 4.0 * B * H * Sx * Sx * dh + 4.0 * rows * D * F,
-                     fusedPrecision="attention fp16 operands (staged), GEMMs fp32 MFMA")
+                     fusedPrecision="attention fp16 operands (staged), GEMMs fp32")
 
 
 # --------------------------------------------------------- timestep embed --

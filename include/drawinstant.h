@@ -255,7 +255,9 @@ int32_t di_layer_norm(di_ctx* ctx, di_handle X, di_handle gamma, di_handle beta,
 
 /* matmul (wgsl-ops.js:477-569, OPS.MatMul wgsl-executor.js:1040-1054):
  * Y[b] = A[b] (M x K) . B (K x N), B batched (offset b*K*N) iff b_batched.
- * fp32 uses fp32 MFMA (exact fp32 products), fp16 the fp16 MFMA. */
+ * fp32 runs on the bf16 MFMA with every operand split into three bf16 parts
+ * (fp32 products and sums, no larger an error than the fp32 MFMA's), fp16 on
+ * the fp16 MFMA. */
 int32_t di_matmul(di_ctx* ctx, di_handle A, di_handle B, di_handle Y, uint32_t M,
                   uint32_t N, uint32_t K, uint32_t batch, int32_t b_batched,
                   int32_t dtype);
@@ -274,7 +276,7 @@ int32_t di_linear(di_ctx* ctx, di_handle X, di_handle W, di_handle bias, di_hand
  * OPS.Conv wgsl-executor.js:1068-1092; batch N >= 1, the reference computes
  * batch 0 only).  Optional residual R (same shape as Y) added after the bias
  * (fused-resnet.js WGSL_CONV :173-208 residual epilogue).
- *   layout DI_NCHW: X NCHW, W OIHW, dtype fp32 (exact fp32 MFMA), or with
+ *   layout DI_NCHW: X NCHW, W OIHW, dtype fp32 (split operands, as di_matmul), or with
  *                   DI_CONV_F16_COMPUTE fp16-in / fp32-acc MFMA;
  *   layout DI_NHWC: X NHWC fp16, W OHWI fp16 ([Cout][K][K][Cin]), Cin % 8 == 0.
  * DI_CONV_UPSAMPLE2X convolves the 2x nearest upsample of X (H, W are X's).

@@ -1,0 +1,128 @@
+"""GPU: the fp32 contractions on the bf16 matrix cores (k_gemm_f32.hip) against
+float64, at the edges of their tiles (64 / 128 rows and columns, 32-deep
+stages), over both operand orders, fp16-resident weights, every convolution
+form and non-finite inputs.
+
+Bound per element: an fp32 sum of K products in any order of at least four
+products per rounding step errs by at most (K / 4 + 16) roundings of 2^-24 of
+sum |a b| (the 16 covers the split's remainder and the last additions)."""
+import numpy as np
+import pytest
+import torch
+import torch.nn.functional as TF
+
+pytestmark = pytest.mark.gpu
+
+F32, F32W16, NCHW = 0, 2, 0
+UP2X, SILU, GEGLU = 2, 4, 2
+
+
+def _call(dev, fn, *a):
+    import drawinstant
+    drawinstant.call(fn, dev.ctx, *a)
+
+
+def _check(got, ref, mag, K, extra=0.0):
+    err = np.abs(got.astype(np.float64) - ref)
+    bound = (K / 4 + 16) * 2.0 ** -24 * mag + 2.0 ** -23 * np.abs(ref) + extra
+    assert got.shape == ref.shape and np.isfinite(got).all()
+    assert (err <= bound).all(), f"{(err / bound).max():.2f} x the bound"
+
+
+def _mats(rng, ash, bsh, scale=1.0, w16=False):
+    a = (rng.standard_normal(ash) * scale).astype(np.float32)
+    b = rng.standard_normal(bsh).astype(np.float32)
+    return a, b.astype(np.float16) if w16 else b
+
+
+@pytest.mark.parametrize("w16", [False, True])
+@pytest.mark.parametrize("trans_b", [0, 1])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (63, 65, 31), (64, 64, 32), (65, 130, 33),
+                                   (129, 127, 100), (3, 1281, 2049), (300, 64, 4100)])
+def test_gemm(dev, rng, M, N, K, trans_b, w16):
+    a, b = _mats(rng, (M, K), (N, K) if trans_b else (K, N), w16=w16)
+    c = rng.standard_normal(N).astype(np.float32)
+    y = dev.create_buffer(M * N * 4)
+    _call(dev, "di_gemm", dev.storage(a).handle, dev.storage(b).handle, dev.storage(c).handle,
+          y.handle, M, N, K, trans_b, F32W16 if w16 else F32)
+    b64 = b.astype(np.float64).T if trans_b else b.astype(np.float64)
+    a64 = a.astype(np.float64)
+    _check(dev.download(y).reshape(M, N), a64 @ b64 + c, np.abs(a64) @ np.abs(b64) + np.abs(c), K)
+
+
+@pytest.mark.parametrize("batched", [0, 1])
+@pytest.mark.parametrize("M,N,K,bt,scale", [(77, 66, 64, 3, 1.0), (40, 77, 130, 5, 2.0 ** -60),
+                                            (128, 64, 257, 2, 2.0 ** 60)])
+def test_matmul(dev, rng, M, N, K, bt, scale, batched):
+    a, b = _mats(rng, (bt, M, K), (bt, K, N) if batched else (K, N), scale)
+    y = dev.create_buffer(bt * M * N * 4)
+    _call(dev, "di_matmul", dev.storage(a).handle, dev.storage(b).handle, y.handle, M, N, K, bt,
+          batched, F32)
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    _check(dev.download(y).reshape(bt, M, N), a64 @ b64, np.abs(a64) @ np.abs(b64), K)
+
+
+@pytest.mark.parametrize("M,N,K", [(70, 96, 40), (33, 32, 1500)])
+def test_linear_geglu_residual(dev, rng, M, N, K):
+    x, w = _mats(rng, (M, K), (N, K))
+    w /= np.float32(np.sqrt(K))
+    b = rng.standard_normal(N).astype(np.float32)
+    r = rng.standard_normal((M, N // 2)).astype(np.float32)
+    y = dev.create_buffer(M * N * 2)
+    _call(dev, "di_linear", dev.storage(x).handle, dev.storage(w).handle, dev.storage(b).handle,
+          dev.storage(r).handle, y.handle, M, N, K, GEGLU, F32)
+    h = x.astype(np.float64) @ w.astype(np.float64).T + b
+    g = h.reshape(M, N // 32, 2, 16)
+    ref = (g[:, :, 0] * TF.gelu(torch.from_numpy(g[:, :, 1])).numpy()).reshape(M, N // 2) + r
+    got = dev.download(y).reshape(M, N // 2)
+    # the GELU's erf polynomial (1.5e-7) times |hidden * gate| dominates
+    assert np.abs(got - ref).max() <= 4e-6 * (1 + np.abs(ref).max())
+
+
+@pytest.mark.parametrize("w16", [False, True])
+@pytest.mark.parametrize("N,ci,co,H,W,k,s,flags", [
+    (1, 3, 5, 9, 11, 3, 1, 0), (2, 64, 70, 8, 8, 3, 2, 0), (1, 67, 65, 13, 10, 1, 1, 0),
+    (3, 33, 64, 5, 7, 3, 1, SILU), (1, 20, 130, 12, 12, 5, 1, 0), (2, 40, 64, 6, 9, 3, 1, UP2X),
+    (1, 300, 64, 16, 8, 3, 1, 0), (1, 7, 3, 20, 20, 7, 3, SILU), (2, 96, 128, 8, 16, 1, 2, 0)])
+def test_conv(dev, rng, N, ci, co, H, W, k, s, flags, w16):
+    x, w = _mats(rng, (N, ci, H, W), (co, ci, k, k), w16=w16)
+    b = rng.standard_normal(co).astype(np.float32)
+
+    def conv(x_, w_, b_):
+        x_ = torch.from_numpy(x_.astype(np.float64))
+        x_ = TF.interpolate(x_, scale_factor=2, mode="nearest") if flags & UP2X else x_
+        return TF.conv2d(x_, torch.from_numpy(w_.astype(np.float64)),
+                         torch.from_numpy(b_.astype(np.float64)), s, k // 2).numpy()
+    z, mag = conv(x, w, b), conv(np.abs(x), np.abs(w), np.abs(b))
+    r = rng.standard_normal(z.shape).astype(np.float32)
+    y = dev.create_buffer(z.size * 4)
+    _call(dev, "di_conv2d", dev.storage(x).handle, dev.storage(w).handle, dev.storage(b).handle,
+          dev.storage(r).handle, y.handle, N, ci, co, H, W, k, s, k // 2, flags,
+          F32W16 if w16 else F32, NCHW)
+    ref = (z / (1 + np.exp(-z)) if flags & SILU else z) + r
+    # SiLU: slope at most 1.1, and a 2-ulp exponential and reciprocal
+    _check(dev.download(y).reshape(z.shape), ref, 1.1 * mag + np.abs(r), ci * k * k,
+           2.0 ** -20 * np.abs(z) if flags & SILU else 0.0)
+
+
+@pytest.mark.parametrize("M,N,K", [(70, 66, 40), (130, 128, 1100)])
+def test_non_finite(dev, rng, M, N, K):
+    """Infinities, NaNs and a value that rounds past bf16's largest follow the
+    fp32 rules (inf * 0 is NaN); rows without them keep the bound."""
+    a, b = _mats(rng, (M, K), (N, K))
+    b[1] = 1.0  # exact in one part: its other parts are zeros
+    a[0, 3], a[2, K - 1], a[5, 7] = np.inf, -np.inf, np.nan
+    a[66, 0] = 3.4e38
+    b[:, 0] *= 1e-3
+    b[4, 3] = 0.0
+    y = dev.create_buffer(M * N * 4)
+    _call(dev, "di_gemm", dev.storage(a).handle, dev.storage(b).handle, 0, y.handle, M, N, K, 1, F32)
+    got = dev.download(y).reshape(M, N)
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        ref, mag = a64 @ b64.T, np.abs(a64) @ np.abs(b64).T
+    bad = ~np.isfinite(ref)
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert np.array_equal(got[bad & ~np.isnan(ref)], ref[bad & ~np.isnan(ref)])
+    rows = [i for i in range(M) if i not in (0, 2, 5)]
+    _check(got[rows], ref[rows], mag[rows], K)
