@@ -202,33 +202,134 @@ __global__ void k_affine_bcast(const T* __restrict__ a, const T* __restrict__ g,
   }
 }
 
-// Transpose: s0 = input strides, s1 = perm (wgsl-ops.js:1019-1031).
+// y = x read through input strides c.s0 of the output's axes: the transposes
+// (wgsl-ops.js:1019-1031) and slices (:1109-1122) that no vector or tile form
+// below takes.
 template <typename T>
-__global__ void k_transpose(const T* __restrict__ x, T* __restrict__ y, Idx4 c, uint64_t n) {
-  uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    uint32_t o[4], in[4] = {0, 0, 0, 0};
-    unravel(c, i, o);
-    for (uint32_t d = 0; d < c.rank; d++) in[c.s1[d]] = o[d];
-    uint64_t off = 0;
-#pragma unroll
-    for (int d = 0; d < 4; d++) off += (uint64_t)in[d] * c.s0[d];
-    y[i] = x[off];
-  }
-}
-
-// Slice: s0 = input strides, s1 = start (wgsl-ops.js:1109-1122).
-template <typename T>
-__global__ void k_slice(const T* __restrict__ x, T* __restrict__ y, Idx4 c, uint64_t n) {
+__global__ void k_gather(const T* __restrict__ x, T* __restrict__ y, Idx4 c, uint64_t n) {
   uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
     uint32_t o[4];
     unravel(c, i, o);
     uint64_t off = 0;
 #pragma unroll
-    for (int d = 0; d < 4; d++) off += (uint64_t)(c.s1[d] + o[d]) * c.s0[d];
+    for (int d = 0; d < 4; d++) off += (uint64_t)o[d] * c.s0[d];
     y[i] = x[off];
   }
+}
+
+// ---- vector forms of the strided ops ----
+// The launcher drops and merges dimensions first (fold_dims), so that most
+// broadcasts are one contiguous run and a head transpose is rows of 64: then
+// a thread moves four elements at a time, with 32-bit coordinates taken once
+// per vector (the element-wise forms above spend up to three 64-bit divisions
+// per element).  Memory bound: a scalar times 5 x 2304 x 2304 scores
+// 73 -> 32 us (6.7 TB/s, partly from the Infinity Cache).
+template <typename T>
+struct Vec4 {
+  typedef T type __attribute__((ext_vector_type(4)));
+};
+
+// Element offsets of vector i (of 4 along the last dimension) in operands
+// with strides c.s0 and c.s1.
+__device__ __forceinline__ void vec_offsets(const Idx4& c, uint32_t i, uint64_t& o0, uint64_t& o1) {
+  o0 = o1 = 0;
+  uint32_t rem = i, n = c.dim[c.rank - 1] / 4;
+  for (int d = (int)c.rank - 1; d > 0; d--) {
+    const uint32_t q = rem / n, r = rem - q * n, e = d == (int)c.rank - 1 ? r * 4 : r;
+    o0 += (uint64_t)e * c.s0[d];
+    o1 += (uint64_t)e * c.s1[d];
+    rem = q;
+    n = c.dim[d - 1];
+  }
+  const uint32_t e = c.rank == 1 ? rem * 4 : rem;
+  o0 += (uint64_t)e * c.s0[0];
+  o1 += (uint64_t)e * c.s1[0];
+}
+
+template <typename T>
+__device__ __forceinline__ typename Vec4<T>::type ld_vec(const T* p, uint32_t inner_stride) {
+  typedef typename Vec4<T>::type V;
+  if (inner_stride) return *(const V*)p;
+  const T v = *p;
+  return V{v, v, v, v};
+}
+
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_binary_bcast_v(int op, const T* __restrict__ a,
+                                                           const T* __restrict__ b,
+                                                           T* __restrict__ y, Idx4 c, uint32_t nv) {
+  typedef typename Vec4<T>::type V;
+  const uint32_t si = c.s0[c.rank - 1], sj = c.s1[c.rank - 1];
+  for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < nv; i += gridDim.x * kBlock) {
+    uint64_t ao, bo;
+    vec_offsets(c, i, ao, bo);
+    const V u = ld_vec<T>(a + ao, si), w = ld_vec<T>(b + bo, sj);
+    V r;
+#pragma unroll
+    for (int j = 0; j < 4; j++) r[j] = (T)binary_op(op, (float)u[j], (float)w[j]);
+    *(V*)(y + (uint64_t)i * 4) = r;
+  }
+}
+
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_affine_bcast_v(const T* __restrict__ a,
+                                                           const T* __restrict__ g,
+                                                           const T* __restrict__ bt,
+                                                           T* __restrict__ y, Idx4 c, uint32_t nv) {
+  typedef typename Vec4<T>::type V;
+  const uint32_t si = c.s0[c.rank - 1], sj = c.s1[c.rank - 1];
+  for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < nv; i += gridDim.x * kBlock) {
+    uint64_t ao, bo;
+    vec_offsets(c, i, ao, bo);
+    const V u = ld_vec<T>(a + ao, si), w = ld_vec<T>(g + bo, sj), z = ld_vec<T>(bt + bo, sj);
+    V r;
+#pragma unroll
+    for (int j = 0; j < 4; j++) r[j] = (T)((float)u[j] * (float)w[j] + (float)z[j]);
+    *(V*)(y + (uint64_t)i * 4) = r;
+  }
+}
+
+// Strided gather of contiguous runs: transposes that keep the last axis, and
+// slices (x already at the slice's start).  s0: input strides of the output's
+// axes.
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_gather_v(const T* __restrict__ x, T* __restrict__ y,
+                                                     Idx4 c, uint32_t nv) {
+  typedef typename Vec4<T>::type V;
+  for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < nv; i += gridDim.x * kBlock) {
+    uint64_t o, unused;
+    vec_offsets(c, i, o, unused);
+    *(V*)(y + (uint64_t)i * 4) = *(const V*)(x + o);
+  }
+}
+
+// Transpose that moves the input's contiguous axis J away from the end:
+// 64 x 64 tiles over (I = the output's last axis, J) through LDS, so reads
+// run along J and writes along I.  Up to two further axes in blockIdx.z.
+// Axes under 16 would leave most of a tile idle: element by element.
+// 4096 x 4096 fp32 60 -> 27 us, 9216 x 512 fp16 22 -> 7.6 us.
+struct TileArgs {
+  uint32_t nI, nJ, n1;   // axis sizes; n1: inner of the two further axes
+  uint64_t sI, oJ;       // input stride of I, output stride of J
+  uint64_t s0, s1, o0, o1;  // further axes: input and output strides
+};
+template <typename T>
+__global__ __launch_bounds__(256) void k_transpose_tile(const T* __restrict__ x, T* __restrict__ y,
+                                                        TileArgs t) {
+  __shared__ T tile[64][65];
+  const uint32_t z0 = blockIdx.z / t.n1, z1 = blockIdx.z % t.n1;
+  const T* xi = x + z0 * t.s0 + z1 * t.s1;
+  T* yo = y + z0 * t.o0 + z1 * t.o1;
+  const uint32_t j0 = blockIdx.x * 64, i0 = blockIdx.y * 64;
+  const uint32_t tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
+#pragma unroll
+  for (uint32_t r = ty; r < 64; r += 4)
+    if (i0 + r < t.nI && j0 + tx < t.nJ) tile[r][tx] = xi[(uint64_t)(i0 + r) * t.sI + j0 + tx];
+  __syncthreads();
+#pragma unroll
+  for (uint32_t r = ty; r < 64; r += 4)
+    if (j0 + r < t.nJ && i0 + tx < t.nI) yo[(uint64_t)(j0 + r) * t.oJ + i0 + tx] = tile[tx][r];
 }
 
 // Striped concat copy (wgsl-ops.js:1142-1157).
@@ -294,43 +395,75 @@ __global__ void k_softmax(const T* __restrict__ x, T* __restrict__ y, uint32_t i
   for (uint32_t j = lane; j < inner; j += kWave) yr[j] = (T)(__expf((float)xr[j] - m) * inv);
 }
 
-// fp16 rows of inner = 512 * NV elements (NV <= 8): one wavefront per row
-// holding the row in registers (NV 16-byte vectors per lane), so the row is
-// read once and written once.
-template <int NV>
-__global__ __launch_bounds__(256) void k_softmax_f16_reg(const f16* __restrict__ x,
-                                                         f16* __restrict__ y, uint32_t rows) {
-  const uint32_t row = blockIdx.x * 4 + threadIdx.x / kWave;
-  const uint32_t lane = threadIdx.x % kWave;
-  if (row >= rows) return;
-  constexpr uint32_t inner = 512 * NV;
-  const f16* xr = x + (uint64_t)row * inner;
-  f16x8 v[NV];
+// Row softmax with the row held in registers: WPR wavefronts per row, each
+// lane NV vectors of VW elements (vector i of lane l at (i * 64 * WPR + l) *
+// VW; elements past the row count as absent), so the row is read and written
+// once, where k_softmax reads it three times.  Memory bound: fp32 11520 rows
+// of 2304 80 -> 31 us (6.9 TB/s, partly from the Infinity Cache), 10240 rows of
+// 77 4.9 -> 4.1 us, fp16 9216 rows of 9216 230 -> 52 us.
+template <typename T, int VW, int NV, int WPR>
+__global__ __launch_bounds__(256) void k_softmax_reg(const T* __restrict__ x, T* __restrict__ y,
+                                                     uint32_t inner, uint32_t rows) {
+  typedef T V __attribute__((ext_vector_type(VW)));
+  __shared__ float red[2][4];
+  const uint32_t wave = threadIdx.x / kWave, lane = threadIdx.x % (kWave * WPR);
+  const uint32_t row = blockIdx.x * (4 / WPR) + wave / WPR;
+  if (row >= rows) return;  // (whole workgroup where WPR = 4)
+  const T* xr = x + (uint64_t)row * inner;
+  float v[NV][VW];
 #pragma unroll
-  for (int i = 0; i < NV; i++) v[i] = *(const f16x8*)(xr + (i * kWave + lane) * 8);
+  for (int i = 0; i < NV; i++) {
+    const uint32_t at = (i * kWave * WPR + lane) * VW;
+    if constexpr (VW == 1) {
+      if (at < inner) v[i][0] = (float)xr[at];
+    } else if (at < inner) {  // inner % VW == 0
+      const V t = *(const V*)(xr + at);
+#pragma unroll
+      for (int e = 0; e < VW; e++) v[i][e] = (float)t[e];
+    }
+  }
   float m = -3.0e38f;
 #pragma unroll
   for (int i = 0; i < NV; i++)
+    if ((i * kWave * WPR + lane) * VW < inner)
 #pragma unroll
-    for (int e = 0; e < 8; e++) m = fmaxf(m, (float)v[i][e]);
+      for (int e = 0; e < VW; e++) m = fmaxf(m, v[i][e]);
   m = wave_max(m);
-  float ex[NV][8], s = 0.0f;
+  if constexpr (WPR > 1) {
+    if (threadIdx.x % kWave == 0) red[0][wave] = m;
+    __syncthreads();
+    m = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));
+  }
+  float s = 0.0f;
 #pragma unroll
   for (int i = 0; i < NV; i++)
+    if ((i * kWave * WPR + lane) * VW < inner)
 #pragma unroll
-    for (int e = 0; e < 8; e++) {
-      ex[i][e] = __expf((float)v[i][e] - m);
-      s += ex[i][e];
-    }
+      for (int e = 0; e < VW; e++) {
+        v[i][e] = __expf(v[i][e] - m);
+        s += v[i][e];
+      }
   s = wave_sum(s);
+  if constexpr (WPR > 1) {
+    if (threadIdx.x % kWave == 0) red[1][wave] = s;
+    __syncthreads();
+    s = (red[1][0] + red[1][1]) + (red[1][2] + red[1][3]);
+  }
   const float inv = 1.0f / s;
-  f16* yr = y + (uint64_t)row * inner;
+  T* yr = y + (uint64_t)row * inner;
 #pragma unroll
   for (int i = 0; i < NV; i++) {
-    f16x8 o;
+    const uint32_t at = (i * kWave * WPR + lane) * VW;
+    if (at < inner) {
+      if constexpr (VW == 1) {
+        yr[at] = (T)(v[i][0] * inv);
+      } else {
+        V o;
 #pragma unroll
-    for (int e = 0; e < 8; e++) o[e] = (f16)(ex[i][e] * inv);
-    *(f16x8*)(yr + (i * kWave + lane) * 8) = o;
+        for (int e = 0; e < VW; e++) o[e] = (T)(v[i][e] * inv);
+        *(V*)(yr + at) = o;
+      }
+    }
   }
 }
 
@@ -442,37 +575,167 @@ uint64_t max_offset(const Idx4& c, const uint32_t* extra_start) {
   return off;
 }
 
+// Drop axes of one element and merge neighbours that both operands walk as
+// one (the outer stride is the inner's times its size, or both are 0).
+// Row-major output order is kept.
+void fold_dims(Idx4* c) {
+  uint32_t r = 0;
+  for (uint32_t d = 0; d < c->rank; d++) {
+    if (c->dim[d] == 1) continue;
+    if (r > 0 && c->s0[r - 1] == (uint64_t)c->s0[d] * c->dim[d] &&
+        c->s1[r - 1] == (uint64_t)c->s1[d] * c->dim[d] &&
+        (uint64_t)c->dim[r - 1] * c->dim[d] < (1ull << 32)) {
+      c->dim[r - 1] *= c->dim[d];
+      c->s0[r - 1] = c->s0[d];
+      c->s1[r - 1] = c->s1[d];
+    } else {
+      c->dim[r] = c->dim[d];
+      c->s0[r] = c->s0[d];
+      c->s1[r] = c->s1[d];
+      r++;
+    }
+  }
+  if (r == 0) {  // one element
+    c->dim[0] = 1;
+    c->s0[0] = c->s1[0] = 0;
+    r = 1;
+  }
+  for (uint32_t d = r; d < 4; d++) {
+    c->dim[d] = 1;
+    c->s0[d] = c->s1[d] = 0;
+  }
+  c->rank = r;
+}
+
+// Whether an operand with strides st allows four-element vectors along the
+// last axis: contiguous there with every other stride and the address a
+// multiple of four elements, or constant there.
+bool vec4_operand(const Idx4& c, const uint32_t* st, const void* p, size_t es) {
+  const uint32_t inner = st[c.rank - 1];
+  if (inner == 0) return true;
+  if (inner != 1 || (uintptr_t)p % (4 * es)) return false;
+  for (uint32_t d = 0; d + 1 < c.rank; d++)
+    if (st[d] % 4) return false;
+  return true;
+}
+
+// Vectors of a folded problem of n elements, or 0 where the vector forms do
+// not apply (a ragged last axis, a misaligned output, over 2^32 vectors less
+// the grid's last step).
+uint32_t vec4_count(const Idx4& c, const void* y, size_t es, uint64_t n) {
+  if (c.dim[c.rank - 1] % 4 || (uintptr_t)y % (4 * es) || n / 4 > 0xf0000000ull) return 0;
+  return (uint32_t)(n / 4);
+}
+
+inline unsigned grid_vec(uint32_t nv) {
+  const uint32_t b = (nv + kBlock - 1) / kBlock;
+  return b < 65536u ? b : 65536u;
+}
+
+// y = x read through input strides c.s0 of the output's axes (c.s1 unused).
+template <typename T>
+void launch_gather(hipStream_t s, const T* x, T* y, Idx4 c, uint64_t n) {
+  for (int d = 0; d < 4; d++) c.s1[d] = c.s0[d];  // (folding looks at both)
+  fold_dims(&c);
+  const uint32_t last = c.rank - 1;
+  const uint32_t nv = vec4_count(c, y, sizeof(T), n);
+  if (nv && c.s0[last] == 1 && vec4_operand(c, c.s0, x, sizeof(T))) {
+    k_gather_v<T><<<grid_vec(nv), kBlock, 0, s>>>(x, y, c, nv);
+    return;
+  }
+  // the input's contiguous axis elsewhere: tiles
+  uint32_t J = c.rank;
+  for (uint32_t d = 0; d < last; d++)
+    if (c.s0[d] == 1) J = d;
+  if (J < last && c.s0[last] != 1 && c.dim[J] >= 16 && c.dim[last] >= 16) {
+    uint64_t out[4];
+    uint64_t o = 1;
+    for (int d = (int)c.rank - 1; d >= 0; d--) {
+      out[d] = o;
+      o *= c.dim[d];
+    }
+    TileArgs t{c.dim[last], c.dim[J], 1, c.s0[last], out[J], 0, 0, 0, 0};
+    uint64_t z = 1;
+    for (uint32_t d = 0; d < last; d++) {
+      if (d == J) continue;
+      if (z == 1) {
+        t.s1 = c.s0[d];
+        t.o1 = out[d];
+        t.n1 = c.dim[d];
+      } else {  // (outer axis first: make it the outer one)
+        t.s0 = t.s1;
+        t.o0 = t.o1;
+        t.s1 = c.s0[d];
+        t.o1 = out[d];
+        t.n1 = c.dim[d];
+      }
+      z *= c.dim[d];
+    }
+    const uint64_t gy = (t.nI + 63) / 64;
+    if (z <= 65535 && gy <= 65535) {
+      k_transpose_tile<T><<<dim3((t.nJ + 63) / 64, (unsigned)gy, (unsigned)z), 256, 0, s>>>(x, y, t);
+      return;
+    }
+  }
+  k_gather<T><<<grid_for(n), kBlock, 0, s>>>(x, y, c, n);
+}
+
 }  // namespace
 
 namespace di {
 
+// Rows are held in registers by one wavefront up to 48 fp32 or 64 fp16 values
+// per lane, above that by the workgroup (fp16 4096: 9.2 us for 4096 rows with
+// one wavefront each, 9.8 with four); rows past 8192 fp32 or 16384 fp16
+// values, and rows past 4096 that 16-byte vectors do not fit, take the
+// three-pass kernel.
+template <typename T>
+static void softmax_dispatch(hipStream_t s, const T* x, T* y, uint32_t inner, uint32_t rows) {
+  constexpr int VW = 16 / (int)sizeof(T);
+  const unsigned g4 = (rows + 3) / 4;
+  const bool vec = (((uintptr_t)x | (uintptr_t)y) & 15) == 0 && inner % VW == 0;
+#define DI_SM(VWV, NVV, WPRV, GRID)                                                  \
+  if (inner <= (uint32_t)(VWV * NVV * WPRV * kWave)) {                               \
+    k_softmax_reg<T, VWV, NVV, WPRV><<<GRID, 256, 0, s>>>(x, y, inner, rows);        \
+    return;                                                                          \
+  }
+  if (vec) {
+    DI_SM(VW, 1, 1, g4)
+    DI_SM(VW, 2, 1, g4)
+    DI_SM(VW, 4, 1, g4)
+    DI_SM(VW, 8, 1, g4)
+    if constexpr (VW == 4) {
+      DI_SM(VW, 12, 1, g4)
+      DI_SM(VW, 4, 4, rows)
+    }
+    DI_SM(VW, 5, 4, rows)
+    DI_SM(VW, 8, 4, rows)
+  } else {
+    DI_SM(1, 2, 1, g4)
+    DI_SM(1, 4, 1, g4)
+    DI_SM(1, 8, 1, g4)
+    DI_SM(1, 16, 1, g4)
+    DI_SM(1, 32, 1, g4)
+    DI_SM(1, 16, 4, rows)
+  }
+#undef DI_SM
+  k_softmax<T><<<g4, 256, 0, s>>>(x, y, inner, rows);
+}
+
 void launch_softmax(hipStream_t s, const void* x, void* y, uint32_t inner, uint32_t rows,
                     int dt) {
   if (rows == 0) return;
-  const unsigned g = (rows + 3) / 4;
-  const bool al16 = (((uintptr_t)x | (uintptr_t)y) & 15) == 0;
-  if (dt == DI_F16 && al16 && inner % 512 == 0 && inner <= 4096) {
-    const f16* xp = (const f16*)x;
-    f16* yp = (f16*)y;
-    switch (inner / 512) {
-      case 1: k_softmax_f16_reg<1><<<g, 256, 0, s>>>(xp, yp, rows); return;
-      case 2: k_softmax_f16_reg<2><<<g, 256, 0, s>>>(xp, yp, rows); return;
-      case 4: k_softmax_f16_reg<4><<<g, 256, 0, s>>>(xp, yp, rows); return;
-      case 8: k_softmax_f16_reg<8><<<g, 256, 0, s>>>(xp, yp, rows); return;
-      default: break;
-    }
-  }
-  if (dt == DI_F32) k_softmax<float><<<g, 256, 0, s>>>((const float*)x, (float*)y, inner, rows);
-  else k_softmax<f16><<<g, 256, 0, s>>>((const f16*)x, (f16*)y, inner, rows);
+  if (dt == DI_F32) softmax_dispatch<float>(s, (const float*)x, (float*)y, inner, rows);
+  else softmax_dispatch<f16>(s, (const f16*)x, (f16*)y, inner, rows);
 }
 
 void launch_transpose_f16(hipStream_t s, const f16* x, uint32_t ldx, uint32_t sx, f16* y,
                           uint32_t batch, uint32_t rows, uint32_t cols) {
   Idx4 c;
-  const uint32_t dim[3] = {batch, cols, rows}, s0[3] = {sx, ldx, 1}, perm[3] = {0, 2, 1};
-  (void)fill_idx4(&c, 3, dim, s0, perm, "launch_transpose_f16");
+  const uint32_t dim[3] = {batch, cols, rows}, s0[3] = {sx, 1, ldx};
+  (void)fill_idx4(&c, 3, dim, s0, s0, "launch_transpose_f16");
   const uint64_t n = (uint64_t)batch * rows * cols;
-  if (n) k_transpose<f16><<<grid_for(n), kBlock, 0, s>>>(x, y, c, n);
+  if (n) launch_gather<f16>(s, x, y, c, n);
 }
 
 }  // namespace di
@@ -573,6 +836,17 @@ int32_t di_binary_bcast(di_ctx* ctx, int32_t op, di_handle A, di_handle B, di_ha
   DI_BUF(ctx, A, a, (max_offset(ca, nullptr) + 1) * dtype_size(dt));
   DI_BUF(ctx, B, b, (max_offset(cb, nullptr) + 1) * dtype_size(dt));
   DI_BUF(ctx, Y, y, numel * dtype_size(dt));
+  fold_dims(&c);
+  const size_t es = dtype_size(dt);
+  const uint32_t nv = vec4_count(c, y->ptr, es, numel);
+  if (nv && vec4_operand(c, c.s0, a->ptr, es) && vec4_operand(c, c.s1, b->ptr, es)) {
+    if (dt == DI_F32)
+      k_binary_bcast_v<float><<<grid_vec(nv), kBlock, 0, ctx->stream>>>(op, (const float*)a->ptr, (const float*)b->ptr, (float*)y->ptr, c, nv);
+    else
+      k_binary_bcast_v<f16><<<grid_vec(nv), kBlock, 0, ctx->stream>>>(op, (const f16*)a->ptr, (const f16*)b->ptr, (f16*)y->ptr, c, nv);
+    DI_LAUNCH_CHECK();
+    return DI_OK;
+  }
   unsigned g = grid_for(numel);
   if (dt == DI_F32)
     k_binary_bcast<float><<<g, kBlock, 0, ctx->stream>>>(op, (const float*)a->ptr, (const float*)b->ptr, (float*)y->ptr, c, numel);
@@ -601,6 +875,18 @@ int32_t di_affine_bcast(di_ctx* ctx, di_handle A, di_handle gamma, di_handle bet
   DI_BUF(ctx, gamma, g_, bc_need);
   DI_BUF(ctx, beta, b_, bc_need);
   DI_BUF(ctx, Y, y, numel * dtype_size(dt));
+  fold_dims(&c);
+  const size_t es = dtype_size(dt);
+  const uint32_t nv = vec4_count(c, y->ptr, es, numel);
+  if (nv && vec4_operand(c, c.s0, a->ptr, es) && vec4_operand(c, c.s1, g_->ptr, es) &&
+      vec4_operand(c, c.s1, b_->ptr, es)) {
+    if (dt == DI_F32)
+      k_affine_bcast_v<float><<<grid_vec(nv), kBlock, 0, ctx->stream>>>((const float*)a->ptr, (const float*)g_->ptr, (const float*)b_->ptr, (float*)y->ptr, c, nv);
+    else
+      k_affine_bcast_v<f16><<<grid_vec(nv), kBlock, 0, ctx->stream>>>((const f16*)a->ptr, (const f16*)g_->ptr, (const f16*)b_->ptr, (f16*)y->ptr, c, nv);
+    DI_LAUNCH_CHECK();
+    return DI_OK;
+  }
   unsigned g = grid_for(numel);
   if (dt == DI_F32)
     k_affine_bcast<float><<<g, kBlock, 0, ctx->stream>>>((const float*)a->ptr, (const float*)g_->ptr, (const float*)b_->ptr, (float*)y->ptr, c, numel);
@@ -677,9 +963,11 @@ int32_t di_transpose(di_ctx* ctx, di_handle X, di_handle Y, uint32_t rank,
   for (uint32_t d = 0; d < rank; d++) maxoff += (uint64_t)(out_dim[d] - 1) * in_stride[perm[d]];
   DI_BUF(ctx, X, x, (maxoff + 1) * dtype_size(dt));
   DI_BUF(ctx, Y, y, numel * dtype_size(dt));
-  unsigned g = grid_for(numel);
-  if (dt == DI_F32) k_transpose<float><<<g, kBlock, 0, ctx->stream>>>((const float*)x->ptr, (float*)y->ptr, c, numel);
-  else k_transpose<f16><<<g, kBlock, 0, ctx->stream>>>((const f16*)x->ptr, (f16*)y->ptr, c, numel);
+  // input strides in the output's axis order
+  Idx4 t = c;
+  for (uint32_t d = 0; d < rank; d++) t.s0[d] = in_stride[perm[d]];
+  if (dt == DI_F32) launch_gather<float>(ctx->stream, (const float*)x->ptr, (float*)y->ptr, t, numel);
+  else launch_gather<f16>(ctx->stream, (const f16*)x->ptr, (f16*)y->ptr, t, numel);
   DI_LAUNCH_CHECK();
   return DI_OK;
 }
@@ -697,9 +985,10 @@ int32_t di_slice(di_ctx* ctx, di_handle X, di_handle Y, uint32_t rank, const uin
   if (numel == 0) return DI_OK;
   DI_BUF(ctx, X, x, (max_offset(c, start) + 1) * dtype_size(dt));
   DI_BUF(ctx, Y, y, numel * dtype_size(dt));
-  unsigned g = grid_for(numel);
-  if (dt == DI_F32) k_slice<float><<<g, kBlock, 0, ctx->stream>>>((const float*)x->ptr, (float*)y->ptr, c, numel);
-  else k_slice<f16><<<g, kBlock, 0, ctx->stream>>>((const f16*)x->ptr, (f16*)y->ptr, c, numel);
+  uint64_t first = 0;  // offset of the slice's start
+  for (uint32_t d = 0; d < rank; d++) first += (uint64_t)start[d] * in_stride[d];
+  if (dt == DI_F32) launch_gather<float>(ctx->stream, (const float*)x->ptr + first, (float*)y->ptr, c, numel);
+  else launch_gather<f16>(ctx->stream, (const f16*)x->ptr + first, (f16*)y->ptr, c, numel);
   DI_LAUNCH_CHECK();
   return DI_OK;
 }
