@@ -28,6 +28,12 @@ struct AttnArgs {
   // key groups inside a workgroup (1 or 2; set by run_attention, only
   // without a split): see k_flash_attn
   uint32_t key_groups = 1;
+  // fp32 tensors: q32 / o32 (strides as q / o, in elements) take the place of
+  // q / o, and k32 / v32 of k / v; null: the fp16 pointers
+  const float* q32 = nullptr;
+  const float* k32 = nullptr;
+  const float* v32 = nullptr;
+  float* o32 = nullptr;
   uint64_t rows = 0;
   f16* part_o = nullptr;
   float* part_ml = nullptr;

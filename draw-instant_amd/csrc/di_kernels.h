@@ -15,6 +15,8 @@ namespace di {
 
 // ---- element-wise / layout (k_eltwise.hip) ----
 void launch_convert(hipStream_t s, const void* src, int sdt, void* dst, int ddt, uint64_t n);
+// Two fp32 tensors of n elements (n % 4 == 0) to fp16, y and y + n, in one launch.
+void launch_convert_pair(hipStream_t s, const float* a, const float* b, f16* y, uint64_t n);
 // [N,C,H,W] layout/dtype change; C_dst >= C pads channels with zeros when the
 // destination is NHWC (used to give conv_in an 8-aligned channel count).
 void launch_layout(hipStream_t s, const void* src, int sdt, int slay, void* dst, int ddt,

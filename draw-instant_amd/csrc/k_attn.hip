@@ -121,7 +121,12 @@ __device__ __forceinline__ float sum_q4(float x) {
 // (max, row sum, output) are merged through LDS at the end.  KS = 1 is the
 // single-group kernel (which may be split over workgroups and merged by
 // k_attn_combine).
-template <int KS>
+//
+// IO: 0 = fp16 tensors; 1 = fp32 queries and outputs (rounded to fp16 as the
+// query fragments are built, stored unrounded); 2 = fp32 keys and values too,
+// which then go through registers into the same LDS image: the next tile's
+// loads are issued at the start of a tile and rounded and stored at its end.
+template <int KS, int IO>
 __global__ __launch_bounds__(256 * KS, 4) void k_flash_attn(AttnArgs a, uint32_t nqb) {
   __shared__ __attribute__((aligned(16))) unsigned char smem[KS * 2 * BUF_BYTES];  // [kg][buf][K | V]
   kernarg_warm(a);
@@ -139,10 +144,11 @@ __global__ __launch_bounds__(256 * KS, 4) void k_flash_attn(AttnArgs a, uint32_t
   const uint32_t qb = w % nqb, rest = w / nqb, split = rest % a.splits, hb = rest / a.splits;
   const uint32_t h = hb % a.H, b = hb / a.H;
 
-  const f16* Q = a.q + b * a.bq + h * a.hq;
-  const f16* K = a.k + b * a.bk + h * a.hk;
-  const f16* V = a.v + b * a.bv + h * a.hv;
-  f16* O = a.o + b * a.bo + h * a.ho;
+  typedef typename std::conditional<IO == 2, float, f16>::type KT;
+  const uint64_t qo = b * a.bq + h * a.hq;
+  const KT* K = (IO == 2 ? (const KT*)a.k32 : (const KT*)a.k) + b * a.bk + h * a.hk;
+  const KT* V = (IO == 2 ? (const KT*)a.v32 : (const KT*)a.v) + b * a.bv + h * a.hv;
+  const uint64_t oo = b * a.bo + h * a.ho;
 
   // Q'^T fragments for the two 32-wide d steps
   const uint32_t qrow = qb * 64 + wave * 16 + r;
@@ -150,7 +156,19 @@ __global__ __launch_bounds__(256 * KS, 4) void k_flash_attn(AttnArgs a, uint32_t
 #pragma unroll
   for (int ks = 0; ks < 2; ks++) {
     f16x8 t = {};
-    if (qrow < a.Sq) t = *(const f16x8*)(Q + (uint64_t)qrow * a.ldq + ks * 32 + g * 8);
+    if (qrow < a.Sq) {
+      const uint64_t at = qo + (uint64_t)qrow * a.ldq + ks * 32 + g * 8;
+      if constexpr (IO == 0) {
+        t = *(const f16x8*)(a.q + at);
+      } else {
+        const f32x4 lo = *(const f32x4*)(a.q32 + at), hi = *(const f32x4*)(a.q32 + at + 4);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          t[j] = (f16)lo[j];
+          t[j + 4] = (f16)hi[j];
+        }
+      }
+    }
 #pragma unroll
     for (int j = 0; j < 8; j++) qf[ks][j] = (f16)((float)t[j] * a.scale_log2);
   }
@@ -160,25 +178,51 @@ __global__ __launch_bounds__(256 * KS, 4) void k_flash_attn(AttnArgs a, uint32_t
   // so it fetches the global chunk (l%8) XOR swizzle(row).  The buffer
   // descriptor of tile t starts at key 64t and ends after the head's last
   // key, so rows past Skv land as zeros.
+  constexpr uint32_t ES = sizeof(KT);
   uint32_t dk[2], dv[2];
 #pragma unroll
   for (int i = 0; i < 2; i++) {
     const uint32_t row = wave * 16 + i * 8 + (lane >> 3), lc = lane & 7;
-    dk[i] = row * (uint32_t)a.ldk * 2u + ((lc ^ ((row >> 1) & 7u)) << 4);
-    dv[i] = row * (uint32_t)a.ldv * 2u + ((lc ^ (row & 7u)) << 4);
+    dk[i] = row * (uint32_t)a.ldk * ES + ((lc ^ ((row >> 1) & 7u)) * (8u * ES));
+    dv[i] = row * (uint32_t)a.ldv * ES + ((lc ^ (row & 7u)) * (8u * ES));
   }
+  f32x4 kr[2][2], vr[2][2];  // IO 2: the tile on its way
   auto dma_kv = [&](int t, auto buf_c) {
     const uint32_t key0 = (uint32_t)t * BKV, left = a.Skv - key0;
     const __amdgpu_buffer_rsrc_t rK =
-        make_rsrc(K + (uint64_t)key0 * a.ldk, (left - 1) * (uint32_t)a.ldk * 2u + D * 2);
+        make_rsrc(K + (uint64_t)key0 * a.ldk, (left - 1) * (uint32_t)a.ldk * ES + D * ES);
     const __amdgpu_buffer_rsrc_t rV =
-        make_rsrc(V + (uint64_t)key0 * a.ldv, (left - 1) * (uint32_t)a.ldv * 2u + D * 2);
+        make_rsrc(V + (uint64_t)key0 * a.ldv, (left - 1) * (uint32_t)a.ldv * ES + D * ES);
     unsigned char* base = smem + (kg * 2 + decltype(buf_c)::value) * BUF_BYTES + wave * 16 * 128;
 #pragma unroll
     for (int i = 0; i < 2; i++) {
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rK, (lds_ptr)(base + i * 8 * 128), 16, dk[i], 0, 0, 0);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rV, (lds_ptr)(base + K_BYTES + i * 8 * 128), 16,
-                                               dv[i], 0, 0, 0);
+      if constexpr (IO == 2) {
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+          kr[i][j] = __builtin_bit_cast(f32x4, buf_load16(rK, dk[i] + 16 * j));
+          vr[i][j] = __builtin_bit_cast(f32x4, buf_load16(rV, dv[i] + 16 * j));
+        }
+      } else {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rK, (lds_ptr)(base + i * 8 * 128), 16, dk[i], 0, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rV, (lds_ptr)(base + K_BYTES + i * 8 * 128), 16,
+                                                 dv[i], 0, 0, 0);
+      }
+    }
+  };
+  // IO 2: the tile that dma_kv fetched, rounded into its buffer
+  auto put_kv = [&](auto buf_c) {
+    unsigned char* base =
+        smem + (kg * 2 + decltype(buf_c)::value) * BUF_BYTES + wave * 16 * 128 + lane * 16;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      f16x8 k8, v8;
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        k8[j] = (f16)kr[i][j >> 2][j & 3];
+        v8[j] = (f16)vr[i][j >> 2][j & 3];
+      }
+      *(f16x8*)(base + i * 8 * 128) = k8;
+      *(f16x8*)(base + K_BYTES + i * 8 * 128) = v8;
     }
   };
 
@@ -288,12 +332,19 @@ __global__ __launch_bounds__(256 * KS, 4) void k_flash_attn(AttnArgs a, uint32_t
       }
     }
     // the next tile has landed in LDS (vmcnt 0), every wave is done with this one
-    __builtin_amdgcn_s_waitcnt(kWaitVm0);
+    if constexpr (IO == 2) {
+      if (t + 1 < t1) put_kv(Int<cur ^ 1>{});
+    } else {
+      __builtin_amdgcn_s_waitcnt(kWaitVm0);
+    }
     __syncthreads();
   };
 
-  if (KS == 1 || t0 < t1) dma_kv(t0, Int<0>{});
-  __builtin_amdgcn_s_waitcnt(kWaitVm0);
+  if (KS == 1 || t0 < t1) {
+    dma_kv(t0, Int<0>{});
+    if constexpr (IO == 2) put_kv(Int<0>{});
+  }
+  if constexpr (IO != 2) __builtin_amdgcn_s_waitcnt(kWaitVm0);
   __syncthreads();
   // two tiles per iteration so each LDS buffer has fixed offsets
   for (int i = 0; i < tpg; i += 2) {
@@ -348,7 +399,13 @@ __global__ __launch_bounds__(256 * KS, 4) void k_flash_attn(AttnArgs a, uint32_t
   }
   if (qrow < a.Sq) {
     const float inv = 1.0f / l;
-    f16* dst = O + (uint64_t)qrow * a.ldo;
+    if (IO > 0 && a.splits == 1) {
+      float* d32 = a.o32 + oo + (uint64_t)qrow * a.ldo;
+#pragma unroll
+      for (int dt = 0; dt < 4; dt++) *(f32x4*)(d32 + dt * 16 + g * 4) = o[dt] * inv;
+      return;
+    }
+    f16* dst = IO > 0 ? nullptr : a.o + oo + (uint64_t)qrow * a.ldo;
     if (a.splits > 1) {
       // this key range's normalised output and (max, row sum), per row
       // (b, h, q) of the [splits][B*H*Sq] workspace
@@ -368,7 +425,7 @@ __global__ __launch_bounds__(256 * KS, 4) void k_flash_attn(AttnArgs a, uint32_t
 
 // Merge the key ranges of a split launch: one thread per 8 outputs (a
 // 16-byte chunk) of a (b, h, q) row; all SP ranges are loaded up front.
-template <int SP>
+template <int SP, bool F32>
 __global__ __launch_bounds__(256) void k_attn_combine(AttnArgs a) {
   kernarg_warm(a);
   const uint32_t i = blockIdx.x * 256 + threadIdx.x, row = i >> 3, c = i & 7;
@@ -394,10 +451,18 @@ __global__ __launch_bounds__(256) void k_attn_combine(AttnArgs a) {
   }
   const float inv = 1.0f / wsum;
   const uint32_t q = row % a.Sq, hb = row / a.Sq, h = hb % a.H, b = hb / a.H;
-  f16x8 out;
+  const uint64_t at = b * a.bo + h * a.ho + (uint64_t)q * a.ldo + c * 8;
+  if constexpr (F32) {
 #pragma unroll
-  for (int j = 0; j < 8; j++) out[j] = (f16)(acc[j] * inv);
-  *(f16x8*)(a.o + b * a.bo + h * a.ho + (uint64_t)q * a.ldo + c * 8) = out;
+    for (int j = 0; j < 8; j += 4)
+      *(f32x4*)(a.o32 + at + j) =
+          f32x4{acc[j] * inv, acc[j + 1] * inv, acc[j + 2] * inv, acc[j + 3] * inv};
+  } else {
+    f16x8 out;
+#pragma unroll
+    for (int j = 0; j < 8; j++) out[j] = (f16)(acc[j] * inv);
+    *(f16x8*)(a.o + at) = out;
+  }
 }
 
 }  // namespace
@@ -443,22 +508,35 @@ uint32_t attn_key_groups(const Ctx* c, uint32_t B, uint32_t H, uint32_t Sq, uint
   return ks;
 }
 
-void launch_attention(const AttnArgs& a, uint32_t B, hipStream_t s) {
+template <int IO>
+static void launch_flash(const AttnArgs& a, uint32_t B, hipStream_t s) {
   const uint32_t nqb = (a.Sq + 63) / 64;
   const dim3 grid(nqb * a.H * B * a.splits);
-  if (a.splits == 1 && a.key_groups == 2) k_flash_attn<2><<<grid, 512, 0, s>>>(a, nqb);
-  else k_flash_attn<1><<<grid, 256, 0, s>>>(a, nqb);
+  if (a.splits == 1 && a.key_groups == 2) k_flash_attn<2, IO><<<grid, 512, 0, s>>>(a, nqb);
+  else k_flash_attn<1, IO><<<grid, 256, 0, s>>>(a, nqb);
+}
+
+template <bool F32>
+static void launch_combine(const AttnArgs& a, hipStream_t s) {
   const dim3 cg((uint32_t)((a.rows * 8 + 255) / 256));
   switch (a.splits) {
     case 1: break;
-    case 2: k_attn_combine<2><<<cg, 256, 0, s>>>(a); break;
-    case 3: k_attn_combine<3><<<cg, 256, 0, s>>>(a); break;
-    case 4: k_attn_combine<4><<<cg, 256, 0, s>>>(a); break;
-    case 5: k_attn_combine<5><<<cg, 256, 0, s>>>(a); break;
-    case 6: k_attn_combine<6><<<cg, 256, 0, s>>>(a); break;
-    case 7: k_attn_combine<7><<<cg, 256, 0, s>>>(a); break;
-    default: k_attn_combine<8><<<cg, 256, 0, s>>>(a); break;
+    case 2: k_attn_combine<2, F32><<<cg, 256, 0, s>>>(a); break;
+    case 3: k_attn_combine<3, F32><<<cg, 256, 0, s>>>(a); break;
+    case 4: k_attn_combine<4, F32><<<cg, 256, 0, s>>>(a); break;
+    case 5: k_attn_combine<5, F32><<<cg, 256, 0, s>>>(a); break;
+    case 6: k_attn_combine<6, F32><<<cg, 256, 0, s>>>(a); break;
+    case 7: k_attn_combine<7, F32><<<cg, 256, 0, s>>>(a); break;
+    default: k_attn_combine<8, F32><<<cg, 256, 0, s>>>(a); break;
   }
+}
+
+void launch_attention(const AttnArgs& a, uint32_t B, hipStream_t s) {
+  if (!a.q32) launch_flash<0>(a, B, s);
+  else if (!a.k32) launch_flash<1>(a, B, s);
+  else launch_flash<2>(a, B, s);
+  if (a.q32) launch_combine<true>(a, s);
+  else launch_combine<false>(a, s);
 }
 
 int run_attention(Ctx* c, AttnArgs a, uint32_t B) {
@@ -554,28 +632,35 @@ int attention_entry(di_ctx* ctx, di_handle Q, di_handle K, di_handle V, di_handl
     DI_LAUNCH_CHECK();
     return DI_OK;
   }
-  // fp32 tensors: stage through fp16 (MFMA operands), write fp32.
-  void *tq = nullptr, *tk = nullptr, *tv = nullptr, *to = nullptr;
-  uint64_t cq, ck, cv, co;
-  int rc = pool_alloc(ctx, nq * 2, &tq, &cq);
-  if (!rc) rc = pool_alloc(ctx, nkv * 2, &tk, &ck);
-  if (!rc) rc = pool_alloc(ctx, nkv * 2, &tv, &cv);
-  if (!rc) rc = pool_alloc(ctx, nq * 2, &to, &co);
-  if (!rc) {
-    launch_convert(ctx->stream, q->ptr, DI_F32, tq, DI_F16, nq);
-    launch_convert(ctx->stream, k->ptr, DI_F32, tk, DI_F16, nkv);
-    launch_convert(ctx->stream, v->ptr, DI_F32, tv, DI_F16, nkv);
-    a.q = (const f16*)tq;
-    a.k = (const f16*)tk;
-    a.v = (const f16*)tv;
-    a.o = (f16*)to;
-    rc = run_attention(ctx, a, B);
-    if (!rc) launch_convert(ctx->stream, to, DI_F16, o->ptr, DI_F32, nq);
+  // fp32 tensors: the kernel rounds queries to its fp16 MFMA operands as it
+  // loads them and stores fp32 outputs.  Keys and values are re-read by every
+  // query block: up to eight 64-key tiles they are rounded as they are staged,
+  // above that by one conversion launch beforehand, so that the tiles keep the
+  // direct path into LDS at half the bytes.  Against three conversions in and
+  // one out around the fp16 kernel: B2 H20 256 x 77 16.4 -> 5.3 us, 512 x 512
+  // (H20) 18.4 -> 8.7, 1024 x 1024 (B2 H10) 28.7 -> 19.9, B2 H5 9216 x 9216
+  // 297 -> 281.
+  a.q32 = (const float*)q->ptr;
+  a.o32 = (float*)o->ptr;
+  // (An output over the keys' or values' own buffer needs them read first.)
+  if (Skv <= 8 * BKV && o->ptr != k->ptr && o->ptr != v->ptr &&
+      (uint64_t)(Skv + BKV) * a.ldk * 4 < (1ull << 31)) {
+    a.k32 = (const float*)k->ptr;
+    a.v32 = (const float*)v->ptr;
+    const int rc = run_attention(ctx, a, B);
+    if (rc) return rc;
+    DI_LAUNCH_CHECK();
+    return DI_OK;
   }
-  if (tq) pool_release(ctx, tq, cq);
-  if (tk) pool_release(ctx, tk, ck);
-  if (tv) pool_release(ctx, tv, cv);
-  if (to) pool_release(ctx, to, co);
+  void* tkv = nullptr;
+  uint64_t cap = 0;
+  int rc = pool_alloc(ctx, nkv * 4, &tkv, &cap);
+  if (rc) return rc;
+  a.k = (const f16*)tkv;
+  a.v = a.k + nkv;
+  launch_convert_pair(ctx->stream, (const float*)k->ptr, (const float*)v->ptr, (f16*)tkv, nkv);
+  rc = run_attention(ctx, a, B);
+  pool_release(ctx, tkv, cap);
   if (rc) return rc;
   DI_LAUNCH_CHECK();
   return DI_OK;

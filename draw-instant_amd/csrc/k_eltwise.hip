@@ -32,6 +32,17 @@ __global__ void k_convert(const S* __restrict__ src, D* __restrict__ dst, uint64
     dst[i] = (D)(float)src[i];
 }
 
+// fp32 a (blockIdx.y 0) and b (1) to fp16 y and y + n; n % 4 == 0.
+__global__ __launch_bounds__(kBlock) void k_convert_pair(const float* __restrict__ a,
+                                                         const float* __restrict__ b,
+                                                         f16* __restrict__ y, uint64_t n) {
+  const float* x = blockIdx.y ? b : a;
+  f16* o = y + (blockIdx.y ? n : 0);
+  for (uint64_t i = ((uint64_t)blockIdx.x * kBlock + threadIdx.x) * 4; i < n;
+       i += (uint64_t)gridDim.x * kBlock * 4)
+    *(f16x4*)(o + i) = __builtin_convertvector(*(const f32x4*)(x + i), f16x4);
+}
+
 // [N,C,HW] <-> [N,HW,C] tile transpose through LDS (64x64 tiles, 256 threads).
 // dir 0: NCHW -> NHWC (dst channel stride C_dst >= C, padded channels zeroed)
 // dir 1: NHWC -> NCHW
@@ -500,6 +511,10 @@ void launch_convert(hipStream_t s, const void* src, int sdt, void* dst, int ddt,
     k_convert<float, float><<<g, kBlock, 0, s>>>((const float*)src, (float*)dst, n);
   else
     k_convert<f16, f16><<<g, kBlock, 0, s>>>((const f16*)src, (f16*)dst, n);
+}
+
+void launch_convert_pair(hipStream_t s, const float* a, const float* b, f16* y, uint64_t n) {
+  k_convert_pair<<<dim3(grid_for(n, 4), 2), kBlock, 0, s>>>(a, b, y, n);
 }
 
 template <typename S, typename D>
