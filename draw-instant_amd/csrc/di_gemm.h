@@ -36,7 +36,9 @@ enum TileCfg {
   // B rows per workgroup of 64x64 K2, so a small-M GEMM spreads its loads
   // over twice the CUs
   TILE_64x32_K2 = 14,
-  TILE_COUNT = 15
+  // 3x3 stride-1 conv on 16 x 16 pixel blocks x 128 channels (k_conv3_big.hip)
+  TILE_CONV3_BIG = 15,
+  TILE_COUNT = 16
 };
 
 struct GemmPlan {
@@ -131,6 +133,15 @@ inline uint32_t gemm_extent(uint64_t bytes) { return bytes < 0x7fff0000ull ? (ui
 // channel chunks writes partials for the split-K reducer).
 bool conv3_halo_ok(const GemmArgs& g);
 void launch_conv3_halo(const GemmArgs& g, hipStream_t s);
+// The large-image conv kernel (TILE_CONV3_BIG, k_conv3_big.hip): whether it
+// takes this NHWC fp16 conv (3x3, stride 1, pad 1, optional 2x nearest
+// upsample, Cin % 64 == 0, Cout % 64 == 0, any image size, no split-K),
+// whether it can write g.stats (images of a multiple of 64 pixels with at most
+// one 16 x 16 block per 64-pixel slot), its tile count and its launch.
+bool conv3_big_ok(const GemmArgs& g);
+bool conv3_big_stats_ok(const GemmArgs& g);
+uint32_t conv3_big_tiles(const GemmArgs& g);
+void launch_conv3_big(const GemmArgs& g, hipStream_t s);
 // The U-Net's conv_in as a direct kernel from the NCHW fp32 latent (4
 // channels) to NHWC fp16 [B*H*W][Cout] (+bias), with GroupNorm statistics
 // per 64-pixel chunk and channel into stats (may be null).  Weights OHWI

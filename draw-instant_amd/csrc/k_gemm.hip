@@ -554,12 +554,12 @@ void launch_splitk_reduce_gn(const GemmArgs& g, const GnFuse& f, hipStream_t s) 
   abort();
 }
 
-const uint32_t kTileM[TILE_COUNT] = {64, 128, 64, 128, 128, 64, 64, 128, 64, 64, 128, 128, 64, 128, 64};
-const uint32_t kTileN[TILE_COUNT] = {64, 64, 128, 128, 160, 160, 64, 64, 128, 128, 64, 128, 64, 64, 32};
+const uint32_t kTileM[TILE_COUNT] = {64, 128, 64, 128, 128, 64, 64, 128, 64, 64, 128, 128, 64, 128, 64, 256};
+const uint32_t kTileN[TILE_COUNT] = {64, 64, 128, 128, 160, 160, 64, 64, 128, 128, 64, 128, 64, 64, 32, 128};
 // Relative per-CU MFMA efficiency of each tile shape (the 2x2 wavefront tile
 // sets LDS bytes per MFMA cycle); tuned by measurement.
 const double kTileEff[TILE_COUNT] = {0.35, 0.5, 0.5, 0.8, 0.85, 0.55, 0.35, 0.5, 0.5,
-                                      0.5, 0.5, 0.8, 0.35, 0.8, 0.25};
+                                      0.5, 0.5, 0.8, 0.35, 0.8, 0.25, 0.8};
 bool vec_epi_ok(const GemmArgs& g, int elem, int tile_cfg);
 
 }  // namespace
@@ -606,7 +606,9 @@ static void env_plan_override(const GemmArgs& g, int elem, const char* env_tile,
     const bool ok = end != env_tile && *end == '\0' && t >= 0 && t < TILE_COUNT &&
                     t != TILE_128x160 &&
                     (t != TILE_CONV3_HALO ||
-                     (conv3_halo_ok(g) && vec_epi_ok(g, elem, TILE_CONV3_HALO)));
+                     (conv3_halo_ok(g) && vec_epi_ok(g, elem, TILE_CONV3_HALO))) &&
+                    (t != TILE_CONV3_BIG ||
+                     (conv3_big_ok(g) && vec_epi_ok(g, elem, TILE_CONV3_BIG)));
     if (ok) plan->tile = (int)t;
   }
   if (env_split) {
@@ -680,6 +682,7 @@ GemmPlan gemm_plan(const GemmArgs& g, int elem, int num_cus) {
   // dominates and the implicit GEMM's larger tiles win); DI_CONV_HALO=0
   // turns it off for A/B runs
   const char* env_halo = getenv("DI_CONV_HALO");
+  GemmPlan halo{-1, 1};
   if (elem == DI_F16 && !env_tile && (!env_halo || atoi(env_halo) != 0) && g.Cin >= 320 &&
       conv3_halo_ok(g) && vec_epi_ok(g, elem, TILE_CONV3_HALO)) {
     // channel-chunk splits bring the workgroup count near 224 (measured best
@@ -693,8 +696,37 @@ GemmPlan gemm_plan(const GemmArgs& g, int elem, int num_cus) {
     }
     const char* env_hs = getenv("DI_CONV_HALO_SPLITS");
     if (env_hs) hs = (uint32_t)atoi(env_hs);
-    if (hs >= 1 && nch % hs == 0) return GemmPlan{TILE_CONV3_HALO, hs};
+    if (hs >= 1 && nch % hs == 0) halo = GemmPlan{TILE_CONV3_HALO, hs};
   }
+  // The large-image conv where its tiles fill a third of the chip and it is the
+  // fastest by these estimates, in microseconds from timings of 22 shapes (us
+  // estimated / measured: 512 -> 512 at 96 x 96 61 / 59, at 192 x 192 61 x 3 /
+  // 183, 128 -> 128 at 768 x 768 185 / 192, 320 -> 320 at 96 x 96 41 / 39): 0.75
+  // a stage of 256 x 128 x 64 and 7 a tile, in whole rounds of 256 workgroups,
+  // against 0.31 a stage of 128 x 64 x 64 for the halo kernel (two per CU: whole
+  // rounds do not show) and 0.72 of 128 x 128 x 64 for the implicit GEMM (0.95
+  // where a workgroup has its CU to itself, split-K where tiles leave CUs idle).
+  // Below that fill the others' smaller tiles win (512 -> 512 at 45 x 66, 60
+  // tiles: 54 against 50 us), and within 8 % the estimates do not tell (960 ->
+  // 320 at 4 x 64 x 64: 108 against 109, measured 105 against 101).  DI_CONV_BIG=0 turns it off for A/B runs.
+  const char* env_big = getenv("DI_CONV_BIG");
+  if (elem == DI_F16 && !env_tile && (!env_big || atoi(env_big) != 0) && conv3_big_ok(g) &&
+      vec_epi_ok(g, elem, TILE_CONV3_BIG)) {
+    const uint32_t tiles = conv3_big_tiles(g);
+    const double stages = g.K / 64.0;
+    const double big = ceil(tiles / 256.0) * (stages * 0.75 + 7.0);
+    double other;
+    if (halo.tile >= 0) {
+      other = std::max(1.0, (double)(g.M / 128) * (g.N / 64) * halo.splits / 256.0) * stages /
+                  halo.splits * 0.31 + 4.0;
+    } else {
+      const uint32_t T = ((g.M + 127) / 128) * ((g.N + 127) / 128), sp = T < 256 ? 256 / T : 1;
+      other = stages / sp * std::max(0.95, 0.72 / 256.0 * T) + 4.0 +
+              (sp > 1 ? 3.0 + (double)g.M * g.N * 4.0 * (sp + 1) / 3.5e6 : 0.0);
+    }
+    if (tiles >= 85 && big < 0.92 * other) return GemmPlan{TILE_CONV3_BIG, 1};
+  }
+  if (halo.tile >= 0) return halo;
   if (elem == DI_F16 && tuned_plan(g, &best)) {
     env_plan_override(g, elem, env_tile, env_split, &best);
     return best;
@@ -708,7 +740,7 @@ GemmPlan gemm_plan(const GemmArgs& g, int elem, int num_cus) {
   double best_t = 1e300;
   for (int tc = 0; tc < TILE_COUNT; tc++) {
     if (tc == TILE_128x160) continue;  // spills registers: not built
-    if (tc >= TILE_64x128_W16) continue;  // sixteen-wave tiles: measured table only
+    if (tc >= TILE_64x128_W16) continue;  // sixteen-wave tiles and conv kernels: chosen above
     if (g.act == ACT_GEGLU && kTileN[tc] == 160) continue;  // GEGLU pairs need even TN
     const uint64_t mt = (g.M + kTileM[tc] - 1) / kTileM[tc], nt = (g.N + kTileN[tc] - 1) / kTileN[tc];
     const uint64_t T = mt * nt * g.batch;
@@ -792,7 +824,8 @@ bool vec_epi_ok(const GemmArgs& g, int elem, int tile_cfg) {
 
 bool gemm_stats_ok(const GemmArgs& g, int elem, int a_mode, int b_mode, int tile_cfg) {
   return gemm_fast_ok(g, elem, a_mode, b_mode) && vec_epi_ok(g, elem, tile_cfg) &&
-         g.act != ACT_GEGLU && g.batch == 1 && (g.splits <= 1 || g.N % 32 == 0);
+         g.act != ACT_GEGLU && g.batch == 1 && (g.splits <= 1 || g.N % 32 == 0) &&
+         (tile_cfg != TILE_CONV3_BIG || conv3_big_stats_ok(g));
 }
 
 bool gemm_rstats_ok(const GemmArgs& g, int elem, int a_mode, int b_mode, int tile_cfg) {
@@ -877,8 +910,18 @@ void launch_gemm(GemmArgs g, int elem, int a_mode, int b_mode, int tile_cfg, hip
       g.vec_epi = vec_epi_ok(g, elem, tile_cfg);
     }
   }
+  bool big = false;
+  if (tile_cfg == TILE_CONV3_BIG) {
+    big = fast && a_mode == A_CONV_NHWC && g.vec_epi && conv3_big_ok(g);
+    if (!big) {
+      tile_cfg = TILE_128x128;
+      g.vec_epi = vec_epi_ok(g, elem, tile_cfg);
+    }
+  }
   if (halo) {
     launch_conv3_halo(g, s);
+  } else if (big) {
+    launch_conv3_big(g, s);
   } else if (fast) {
     if (a_mode == A_DENSE && g.ln_rows && g.splits <= 1) gemm_fast_dense_ex(g, tile_cfg, s);
     else if (a_mode == A_DENSE && g.rstats) gemm_fast_dense_ex(g, tile_cfg, s);
