@@ -653,6 +653,14 @@ __global__ __launch_bounds__(64 * WGM * WGN * KS) void k_gemm(GemmArgs g) {
   // Tile order: N fastest, so consecutive tiles share A rows.  Workgroups are
   // dealt round-robin to the 8 XCDs (each with its own L2); remap so that
   // each XCD gets a contiguous run of tiles and shares their A / B reads.
+  // Where B is past the XCD's 4 MiB of L2 the run goes down blocks of 8 tile
+  // rows, column by column: the 64 or so tiles an XCD has in flight then cover
+  // 8 x 8 tiles, not one row that reads all of B again for every tile row
+  // (64 x 128 tiles: 1165 x 10240 x 1280 80 -> 50 us, 7027 x 5120 x 1280 192 ->
+  // 138; 128 x 128: 5120 x 5120 x 640 61 -> 56, 7027 x 5120 x 1280 142 -> 129;
+  // 256 x 10240 x 1280 20 -> 15.5).  Blocks of 4 rows lose 2-5 % to 8 and of 16
+  // gain nothing; a B that the L2 holds is best read row by row (1260 x 1920 x
+  // 640 and its transformer block in blocks: 2 % slower).
   const uint32_t n_tiles = (g.N + BN - 1) / BN;
   const uint32_t n_wg = gridDim.x;
   uint32_t tile = blockIdx.x;
@@ -660,7 +668,14 @@ __global__ __launch_bounds__(64 * WGM * WGN * KS) void k_gemm(GemmArgs g) {
     const uint32_t per = n_wg / 8, rem = n_wg % 8, xcd = tile % 8, slot = tile / 8;
     tile = xcd < rem ? xcd * (per + 1) + slot : rem * (per + 1) + (xcd - rem) * per + slot;
   }
-  const uint32_t m0 = (tile / n_tiles) * BM, n0 = (tile % n_tiles) * BN;
+  uint32_t tm = tile / n_tiles, tn = tile % n_tiles;
+  if (n_tiles > 8 && (uint64_t)g.N * g.k_split * sizeof(TB) > 4u << 20) {
+    const uint32_t t0 = tm & ~7u, in = (tm - t0) * n_tiles + tn;
+    const uint32_t rows = min((g.M + BM - 1) / BM - t0, 8u);
+    tn = in / rows;
+    tm = t0 + in % rows;
+  }
+  const uint32_t m0 = tm * BM, n0 = tn * BN;
   const uint32_t splits = g.splits;
   const uint32_t bz = blockIdx.z / splits, split = blockIdx.z % splits;
   const uint32_t k_begin = split * g.k_split;
