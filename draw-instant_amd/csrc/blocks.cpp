@@ -23,6 +23,14 @@ namespace di {
 
 namespace {
 
+// The reducer's records of the context's statistics-exchange area, which
+// splitk_gn_ok's answer depends on.
+void gn_exchange_area(Ctx* c, GnFuse& f) {
+  f.xchg = c->gn_xchg ? (uint64_t*)c->gn_xchg + (uint64_t)kXchgNchwRecs * kXchgWords : nullptr;
+  const char* e_spin = getenv("DI_GN_XCHG_SPIN");  // 0 forces the recomputing path
+  f.spin = e_spin ? (uint32_t)strtoul(e_spin, nullptr, 10) : 20000u;
+}
+
 int run(Ctx* c, GemmArgs& g, int a_mode, StatsOut* st = nullptr, RowStatsOut* rst = nullptr,
         GnFuseOut* gn = nullptr) {
   const GemmPlan plan = gemm_plan(g, DI_F16, c->num_cus);
@@ -31,11 +39,7 @@ int run(Ctx* c, GemmArgs& g, int a_mode, StatsOut* st = nullptr, RowStatsOut* rs
   g.stats = nullptr;
   g.rstats = nullptr;
   if (gn) {
-    // the reducer's records of the context's statistics-exchange area
-    gn->f.xchg = c->gn_xchg ? (uint64_t*)c->gn_xchg + (uint64_t)kXchgNchwRecs * kXchgWords
-                            : nullptr;
-    const char* e_spin = getenv("DI_GN_XCHG_SPIN");  // 0 forces the recomputing path
-    gn->f.spin = e_spin ? (uint32_t)strtoul(e_spin, nullptr, 10) : 20000u;
+    gn_exchange_area(c, gn->f);
     gn->done = splitk_gn_ok(g, gn->f);
   }
   if (st) st->done = false;
@@ -63,7 +67,7 @@ int run(Ctx* c, GemmArgs& g, int a_mode, StatsOut* st = nullptr, RowStatsOut* rs
   DI_REQUIRE(!g.ln_rows || gemm_lnfold_ok(g, DI_F16, tile), DI_EUNSUPPORTED,
              "LayerNorm fold needs the vector epilogue (M=%u N=%u K=%u tile %d)", g.M, g.N, g.K,
              tile);
-  if (g.splits > 1) {
+  if (g.splits > 1 || g.part_only) {
     void* ws = nullptr;
     int rc = workspace(c, gemm_ws_bytes(g), &ws);
     if (rc) return rc;
@@ -71,7 +75,7 @@ int run(Ctx* c, GemmArgs& g, int a_mode, StatsOut* st = nullptr, RowStatsOut* rs
   }
   if (gn && gn->done) g.part_cpg = g.N / gn->f.groups;
   if (g.splits <= 1) {
-    DI_REQUIRE(!g.part_only && !g.part_slots, DI_EINVAL,
+    DI_REQUIRE(g.part_only || !g.part_slots, DI_EINVAL,
                "shared partial slots need a plan that splits (M=%u N=%u K=%u)", g.M, g.N, g.K);
   }
   launch_gemm(g, DI_F16, a_mode, B_NK, tile, c->stream, gn && gn->done ? &gn->f : nullptr);
@@ -289,20 +293,29 @@ int resnet_forward(Ctx* c, const ResnetW& w, const ResnetShape& s, NhwcSrc x, co
     k1.pad = 0;
     k1.w = w.sk_w;
     k1.bias = w.sk_b;
-    // Both split: the shortcut writes its partials into slots after
-    // conv2's, launches no reducer, and conv2's reducer sums every slot
-    // with the summed bias (conv2 + shortcut = one sum over both k ranges)
+    // conv2 splits: the shortcut writes its sums (one slot where it does not
+    // split itself) into slots after conv2's, launches no reducer, and conv2's
+    // reducer sums every slot with the summed bias (conv2 + shortcut = one
+    // fp32 sum over both k ranges).  A lone slot that takes conv2's GroupNorm
+    // out of its reducer is not worth the launch it costs.
     const GemmPlan pk = conv_plan(c, k1), p2 = conv_plan(c, c2);
-    if (w.c2sk_b && !sk_partials_off() && pk.splits > 1 && p2.splits > 1) {
-      const uint32_t slots = pk.splits + p2.splits;
+    const uint32_t slots = pk.splits + p2.splits;
+    if (c2.gn) gn_exchange_area(c, c2.gn->f);
+    auto gn_fuses = [&](uint32_t part_slots, const float* bias) {
+      ConvCall cc = c2;
+      cc.part_slots = part_slots;
+      cc.bias = bias;
+      GemmArgs g2 = conv_args(cc);
+      g2.splits = p2.splits;
+      return cc.gn && splitk_gn_ok(g2, cc.gn->f);
+    };
+    const bool fused = gn_fuses(slots, w.c2sk_b);
+    if (w.c2sk_b && !sk_partials_off() && p2.splits > 1 &&
+        (pk.splits > 1 || fused || !gn_fuses(0, w.c2_b))) {
       c2.bias = w.c2sk_b;
       c2.part_slots = slots;
-      if (c2.gn) {
-        // the fused GroupNorm reducer reads the partials in column groups
-        GemmArgs g2 = conv_args(c2);
-        g2.splits = p2.splits;
-        if (splitk_gn_ok(g2, c2.gn->f)) k1.part_cpg = s.Cout / c2.gn->f.groups;
-      }
+      // the fused GroupNorm reducer reads the partials in column groups
+      if (fused) k1.part_cpg = s.Cout / c2.gn->f.groups;
       k1.part_slot0 = p2.splits;
       k1.part_slots = slots;
       k1.part_only = 1;

@@ -90,8 +90,9 @@ struct GemmArgs {
   // Partials shared with another launch (a ResNet's 1x1 shortcut and its
   // conv2): this launch writes slots part_slot0 + split of a buffer of
   // part_slots slots ([part_slots][batch][M][N]; 0: its own splits);
-  // part_only = 1 launches no reducer (a later launch's reducer sums every
-  // slot), else the reducer sums all part_slots slots.
+  // part_only = 1 writes slots also without a split and launches no reducer
+  // (a later launch's reducer sums every slot), else the reducer sums all
+  // part_slots slots.
   uint32_t part_slot0 = 0, part_slots = 0;
   int part_only = 0;
   // Optional GroupNorm statistics of the stored output (see gemm_stats_ok):
@@ -120,7 +121,7 @@ struct GemmArgs {
 
 // Tile shape and split-K factor from a cost model (env DI_GEMM_TILE /
 // DI_GEMM_SPLITS override, for tuning sweeps).
-GemmPlan gemm_plan(const GemmArgs& g, int elem, int num_cus);
+GemmPlan gemm_plan(const GemmArgs& g, int elem, int num_cus, int b_mode = B_NK);
 uint64_t gemm_ws_bytes(const GemmArgs& g);
 // Whether the buffer-load (FAST) kernel variant applies.
 bool gemm_fast_ok(const GemmArgs& g, int elem, int a_mode, int b_mode);

@@ -661,7 +661,111 @@ static GemmPlan f32_plan(const GemmArgs& g, int num_cus) {
   return best;
 }
 
-GemmPlan gemm_plan(const GemmArgs& g, int elem, int num_cus) {
+namespace {
+
+// Plan of an fp16 problem of the buffer-load kernels from what their tiles
+// measure on a MI355X: microseconds per 64-deep stage of a workgroup that has
+// its CU to itself (`alone`: barriers and LDS round trips in series) and of
+// each of the several that a CU holds (`shared`), the epilogue of each
+// workgroup after a CU's first (`epi`) and the launch with the first one's
+// prologue and epilogue (`base`), for dense operands and for convolutions
+// (whose loads add address work per stage); a split adds its reducer.  Fitted
+// to 9700 timings, every tile and 1-16 splits of 124 dense shapes (64 to 16384
+// rows, K 64 to 5120) and 85 convolutions (1x1 and 3x3, strided and upsampled,
+// 64 to 1920 channels, 8 to 128 pixels a side): its choices take 1.011 of the
+// best plan's time on average and 1.12 at most, where one efficiency per tile
+// and a fixed 1.25 us a workgroup in whole rounds of the chip took 1.17 and
+// 1.52 (5120 x 640 x 2560: 34 -> 26 us; 1280 -> 640 3x3 at 46 x 118: 158 ->
+// 106; 512 -> 512 3x3 at 2 x 80 x 28: 61 -> 42).  The 64-row tiles of sixteen
+// waves never won and are left to the tuned plans.
+struct TileTime {
+  int id;
+  double alone, shared, epi, base;
+};
+
+GemmPlan f16_plan(const GemmArgs& g, int num_cus, double* est_us = nullptr) {
+  static const TileTime dense[] = {{TILE_64x64, 0.23, 0.197, 0.45, 4.3},
+                                   {TILE_128x64, 0.40, 0.336, 0.9, 5.2},
+                                   {TILE_64x128, 0.38, 0.317, 0.95, 5.1},
+                                   {TILE_128x128, 0.38, 0.585, 1.55, 6.6},
+                                   {TILE_64x64_K2, 0.15, 0.175, 0.85, 4.35},
+                                   {TILE_128x64_K2, 0.31, 0.303, 1.35, 4.85},
+                                   {TILE_64x128_K2, 0.02, 0.302, 1.3, 5.0},
+                                   {TILE_128x64_W16, 0.29, 0.31, 3.0, 4.85},
+                                   {TILE_128x128_W16, 0.06, 0.473, 5.5, 6.1},
+                                   {TILE_64x32_K2, 0.11, 0.123, 0.5, 4.35}};
+  static const TileTime conv[] = {{TILE_64x64, 0.30, 0.198, 0.15, 5.45},
+                                  {TILE_128x64, 0.51, 0.341, 0.9, 6.1},
+                                  {TILE_64x128, 0.45, 0.323, 0.25, 6.0},
+                                  {TILE_128x128, 0.70, 0.484, 1.1, 7.1},
+                                  {TILE_64x64_K2, 0.23, 0.188, 0.75, 5.1},
+                                  {TILE_128x64_K2, 0.39, 0.298, 1.0, 5.7},
+                                  {TILE_64x128_K2, 0.33, 0.292, 0.8, 5.7},
+                                  {TILE_128x64_W16, 0.01, 0.36, 2.7, 5.95},
+                                  {TILE_128x128_W16, 0.03, 0.496, 4.0, 7.0},
+                                  {TILE_64x32_K2, 0.22, 0.144, 0.5, 5.05}};
+  const bool is_conv = g.Cin > 0 && g.ks > 1;
+  const uint32_t stages = g.K / 64;
+  GemmPlan best{TILE_64x64, 1};
+  double best_t = 1e300;
+  for (int i = 0; i < 10; i++) {
+    const TileTime& t = is_conv ? conv[i] : dense[i];
+    // 16 columns to a wave: only the vector epilogue pairs GEGLU's columns
+    if (t.id == TILE_64x32_K2 && g.act == ACT_GEGLU && !vec_epi_ok(g, DI_F16, t.id)) continue;
+    const uint64_t T =
+        (uint64_t)((g.M + kTileM[t.id] - 1) / kTileM[t.id]) * ((g.N + kTileN[t.id] - 1) / kTileN[t.id]) * g.batch;
+    for (uint32_t s = 1; s <= 32; s++) {
+      const uint32_t per = (stages + s - 1) / s;
+      if (s > 1 && per < 2) break;
+      if (s > 1 && (stages + per - 1) / per != s) continue;  // an empty split
+      const uint64_t w = (T * s + num_cus - 1) / num_cus;  // workgroups of the fullest CU
+      double us = t.base + per * std::max(t.alone, w * t.shared) + (double)(w - 1) * t.epi;
+      if (s > 1) us += 2.5 + 0.1 * s + (double)g.batch * g.M * g.N * 4.0 * (s + 1) / 4.0e6;
+      if (us < best_t) {
+        best_t = us;
+        best = GemmPlan{t.id, s};
+      }
+    }
+  }
+  if (est_us) *est_us = best_t;
+  return best;
+}
+
+// Plan of the bounds-checked fp16 kernels (a K that is no multiple of 64,
+// operands of unknown extent or past 31-bit offsets, B stored K x N): the two
+// tile shapes behind the plan's names by one efficiency each.
+GemmPlan slow_plan(const GemmArgs& g, int num_cus) {
+  const double cus = num_cus;
+  GemmPlan best{TILE_64x64, 1};
+  double best_t = 1e300;
+  for (int tc = 0; tc < TILE_COUNT; tc++) {
+    if (tc == TILE_128x160) continue;  // spills registers: not built
+    if (tc >= TILE_64x128_W16) continue;  // sixteen-wave tiles and conv kernels: chosen above
+    if (g.act == ACT_GEGLU && kTileN[tc] == 160) continue;  // GEGLU pairs need even TN
+    const uint64_t mt = (g.M + kTileM[tc] - 1) / kTileM[tc], nt = (g.N + kTileN[tc] - 1) / kTileN[tc];
+    const uint64_t T = mt * nt * g.batch;
+    for (uint32_t s = 1; s <= 32; s++) {
+      const uint32_t kper = ((g.K + s - 1) / s + 63) / 64 * 64;
+      if (s > 1 && kper < 256) break;
+      const double rounds = ceil((double)T * s / cus);
+      // cycles per work unit at the tile's efficiency (4096 fp16 FLOP/clk/CU)
+      // plus a fixed prologue / epilogue cost
+      const double cyc = 2.0 * kTileM[tc] * kTileN[tc] * kper / (4096.0 * kTileEff[tc]) + 3000.0;
+      double t = rounds * cyc;
+      if (s > 1)  // fp32 partials written and read back (~4 TB/s) plus a launch
+        t += (double)g.batch * g.M * g.N * 4.0 * (s + 1) / (4.0e12 / 2.4e9) + 5000.0;
+      if (t < best_t * 0.97) {
+        best_t = t;
+        best = GemmPlan{tc, s};
+      }
+    }
+  }
+  return best;
+}
+
+}  // namespace
+
+GemmPlan gemm_plan(const GemmArgs& g, int elem, int num_cus, int b_mode) {
   // DI_GEMM_PLAN="M,N,K,tile,splits;..." fixes the plan of the listed fp16
   // shapes only (tuning runs of the whole step; tile 13 = the halo conv)
   if (const char* env_plan = getenv("DI_GEMM_PLAN"); env_plan && elem == DI_F16) {
@@ -704,11 +808,12 @@ GemmPlan gemm_plan(const GemmArgs& g, int elem, int num_cus) {
   // 183, 128 -> 128 at 768 x 768 185 / 192, 320 -> 320 at 96 x 96 41 / 39): 0.75
   // a stage of 256 x 128 x 64 and 7 a tile, in whole rounds of 256 workgroups,
   // against 0.31 a stage of 128 x 64 x 64 for the halo kernel (two per CU: whole
-  // rounds do not show) and 0.72 of 128 x 128 x 64 for the implicit GEMM (0.95
-  // where a workgroup has its CU to itself, split-K where tiles leave CUs idle).
-  // Below that fill the others' smaller tiles win (512 -> 512 at 45 x 66, 60
-  // tiles: 54 against 50 us), and within 8 % the estimates do not tell (960 ->
-  // 320 at 4 x 64 x 64: 108 against 109, measured 105 against 101).  DI_CONV_BIG=0 turns it off for A/B runs.
+  // rounds do not show) and the implicit GEMM's own plan.  Below that fill the
+  // others' smaller tiles win (512 -> 512 at 45 x 66, 60 tiles: 54 against 50
+  // us).  At these sizes the big kernel measures 0.93 of its estimate and the
+  // others 1.1 of theirs, hence the factor: over 110 more shapes the choice then
+  // takes 1.003 of the faster kernel's time on average and 1.13 at most (with
+  // equal estimates 1.012 and 1.35).  DI_CONV_BIG=0 turns it off for A/B runs.
   const char* env_big = getenv("DI_CONV_BIG");
   if (elem == DI_F16 && !env_tile && (!env_big || atoi(env_big) != 0) && conv3_big_ok(g) &&
       vec_epi_ok(g, elem, TILE_CONV3_BIG)) {
@@ -720,11 +825,9 @@ GemmPlan gemm_plan(const GemmArgs& g, int elem, int num_cus) {
       other = std::max(1.0, (double)(g.M / 128) * (g.N / 64) * halo.splits / 256.0) * stages /
                   halo.splits * 0.31 + 4.0;
     } else {
-      const uint32_t T = ((g.M + 127) / 128) * ((g.N + 127) / 128), sp = T < 256 ? 256 / T : 1;
-      other = stages / sp * std::max(0.95, 0.72 / 256.0 * T) + 4.0 +
-              (sp > 1 ? 3.0 + (double)g.M * g.N * 4.0 * (sp + 1) / 3.5e6 : 0.0);
+      f16_plan(g, num_cus, &other);
     }
-    if (tiles >= 85 && big < 0.92 * other) return GemmPlan{TILE_CONV3_BIG, 1};
+    if (tiles >= 85 && big < 1.1 * other) return GemmPlan{TILE_CONV3_BIG, 1};
   }
   if (halo.tile >= 0) return halo;
   if (elem == DI_F16 && tuned_plan(g, &best)) {
@@ -736,30 +839,8 @@ GemmPlan gemm_plan(const GemmArgs& g, int elem, int num_cus) {
     env_plan_override(g, elem, env_tile, env_split, &best);
     return best;
   }
-  const double cus = num_cus;
-  double best_t = 1e300;
-  for (int tc = 0; tc < TILE_COUNT; tc++) {
-    if (tc == TILE_128x160) continue;  // spills registers: not built
-    if (tc >= TILE_64x128_W16) continue;  // sixteen-wave tiles and conv kernels: chosen above
-    if (g.act == ACT_GEGLU && kTileN[tc] == 160) continue;  // GEGLU pairs need even TN
-    const uint64_t mt = (g.M + kTileM[tc] - 1) / kTileM[tc], nt = (g.N + kTileN[tc] - 1) / kTileN[tc];
-    const uint64_t T = mt * nt * g.batch;
-    for (uint32_t s = 1; s <= 32; s++) {
-      const uint32_t kper = ((g.K + s - 1) / s + 63) / 64 * 64;
-      if (s > 1 && kper < 256) break;
-      const double rounds = ceil((double)T * s / cus);
-      // cycles per work unit at the tile's efficiency (4096 fp16 FLOP/clk/CU)
-      // plus a fixed prologue / epilogue cost
-      const double cyc = 2.0 * kTileM[tc] * kTileN[tc] * kper / (4096.0 * kTileEff[tc]) + 3000.0;
-      double t = rounds * cyc;
-      if (s > 1)  // fp32 partials written and read back (~4 TB/s) plus a launch
-        t += (double)g.batch * g.M * g.N * 4.0 * (s + 1) / (4.0e12 / 2.4e9) + 5000.0;
-      if (t < best_t * 0.97) {
-        best_t = t;
-        best = GemmPlan{tc, s};
-      }
-    }
-  }
+  const bool fast = gemm_fast_ok(g, elem, g.Cin > 0 ? A_CONV_NHWC : A_DENSE, b_mode);
+  best = fast ? f16_plan(g, num_cus) : slow_plan(g, num_cus);
   env_plan_override(g, elem, env_tile, env_split, &best);
   return best;
 }
@@ -796,7 +877,7 @@ void launch_repack_oihw_ohwi(hipStream_t s, const void* w, int wdt, void* out, u
 
 uint64_t gemm_ws_bytes(const GemmArgs& g) {
   const uint64_t slots = g.part_slots ? g.part_slots : g.splits;
-  return g.splits > 1 ? slots * g.batch * g.M * g.N * sizeof(float) : 0;
+  return slots > 1 ? slots * g.batch * g.M * g.N * sizeof(float) : 0;
 }
 
 bool gemm_fast_ok(const GemmArgs& g, int elem, int a_mode, int b_mode) {
@@ -933,7 +1014,7 @@ void launch_gemm(GemmArgs g, int elem, int a_mode, int b_mode, int tile_cfg, hip
   } else {
     gemm_slow(g, elem, a_mode, b_mode, tile_cfg, s);
   }
-  if (g.splits > 1 && g.part_only) return;  // a later launch's reducer sums the slots
+  if (g.part_only) return;  // a later launch's reducer sums the slots
   if (g.splits > 1 && g.part_slots) g.splits = g.part_slots;  // the reducers sum every slot
   if (g.splits > 1 && gn) {
     launch_splitk_reduce_gn(g, *gn, s);  // g.part_cpg set by the caller

@@ -341,7 +341,7 @@ __device__ __forceinline__ void epi_load_geglu(const GemmArgs& g, uint32_t m0, u
 template <int BM, int BN, int NT>
 __device__ __forceinline__ void epi_prefetch(const GemmArgs& g, uint32_t m0, uint32_t n0, uint32_t bz,
                                              EpiOps<BM, BN, NT>& o) {
-  if (g.splits > 1 || g.act == ACT_GEGLU) return;
+  if (g.splits > 1 || g.part_only || g.act == ACT_GEGLU) return;
   epi_load<BM, BN, NT>(g, m0, n0, bz, 0, o);
 }
 
@@ -367,7 +367,7 @@ __device__ __forceinline__ void gemm_epilogue_vec(const GemmArgs& g, const float
     for (int t = 1; t < NSUM; t++) v += ld4(&sC[i + t * tstride]);
     return v;
   };
-  if (g.splits > 1) {
+  if (g.splits > 1 || g.part_only) {
     constexpr int VPR4 = BN / 4;
     constexpr int NV = (BM * VPR4 + NT - 1) / NT;
     float* P = g.part + ((uint64_t)(split + g.part_slot0) * g.batch + bz) * (uint64_t)g.M * g.N;
@@ -1158,7 +1158,7 @@ __global__ __launch_bounds__(64 * WGM * WGN * KS) void k_gemm(GemmArgs g) {
 #pragma unroll
         for (int i = 0; i < 4; i++) acc[a][b][i] += sC[(wm0 + a * 16 + rq + i) * LDC + wn0 + b * 16 + fr];
   }
-  if (splits > 1) {
+  if (splits > 1 || g.part_only) {
     float* P = g.part + ((uint64_t)(split + g.part_slot0) * g.batch + bz) * (uint64_t)g.M * g.N;
 #pragma unroll
     for (int a = 0; a < TM; a++)

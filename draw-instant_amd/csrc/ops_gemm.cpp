@@ -10,7 +10,7 @@ namespace {
 
 int run_gemm(di_ctx* ctx, GemmArgs& g, int elem, int a_mode, int b_mode, int tile = -1,
              int splits = -1) {
-  const GemmPlan plan = gemm_plan(g, elem, ctx->num_cus);
+  const GemmPlan plan = gemm_plan(g, elem, ctx->num_cus, b_mode);
   if (tile < 0) tile = plan.tile;
   g.splits = splits > 0 ? (uint32_t)splits : plan.splits;
   if (g.splits > 1) {
