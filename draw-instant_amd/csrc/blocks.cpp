@@ -219,7 +219,7 @@ int resnet_forward(Ctx* c, const ResnetW& w, const ResnetShape& s, NhwcSrc x, co
   const uint32_t HW = s.H * s.W;
   const uint64_t rows = (uint64_t)s.B * HW;
   // conv1 hands GN2 the statistics of its output (no partial pass)
-  const bool st2 = HW % 64 == 0;
+  const bool st2 = gn_stats_chunks_ok(s.B, HW);
   Scratch t1, t2, t3, sk, t2st;
   int rc = x_gn ? 0 : t1.alloc(c, rows * s.Cin * 2);
   if (!rc) rc = t2.alloc(c, rows * s.Cout * 2);

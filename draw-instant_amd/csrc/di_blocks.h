@@ -107,7 +107,7 @@ struct ResnetShape {
 // image, temb[b * ld_temb + c] (already offset to this block), may be null.
 // x_st: GroupNorm statistics of x from its producer (null: GN1 computes
 // them); out_st: if non-null, asks for out's statistics ([B*HW/64][Cout]
-// pairs, see GnStats; needs HW % 64 == 0) and reports whether they were
+// pairs, see GnStats; where gn_stats_chunks_ok) and reports whether they were
 // written.  out_gn: if non-null, asks conv2's split-K reducer to apply the
 // next block's GroupNorm to out as well (GnFuse with raw = 1) and reports
 // whether it did; out's statistics are then written only where
@@ -201,7 +201,7 @@ int linear_f16(Ctx* c, const f16* x, uint64_t ldx, uint32_t M, uint32_t K, const
                uint64_t ldy, StatsOut* stats = nullptr, RowStatsOut* rstats = nullptr,
                const LnFold* ln = nullptr);
 
-// Floats of the GroupNorm statistics of a [rows][C] output (rows % 64 == 0).
-inline uint64_t gn_stats_floats(uint64_t rows, uint32_t C) { return rows / 64 * C * 2; }
+// Floats of the GroupNorm statistics of a [rows][C] output.
+inline uint64_t gn_stats_floats(uint64_t rows, uint32_t C) { return (rows + 63) / 64 * C * 2; }
 
 }  // namespace di

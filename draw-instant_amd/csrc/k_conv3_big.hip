@@ -345,7 +345,7 @@ __global__ __launch_bounds__(512, 2) void k_conv3_big(GemmArgs g) {
         sm[b][i] = row_sum16(sm[b][i]);
         sq[b][i] = row_sum16(sq[b][i]);
       }
-    const uint32_t slots = g.Ho * g.Wo / 64, nblk = nby * nbx;
+    const uint32_t slots = (g.Ho * g.Wo + 63) / 64, nblk = nby * nbx;
     float* st = g.stats + (uint64_t)T.img * slots * g.N * 2;
     if (slots == 4 * nblk) {  // whole blocks: one slot per wave
       if (r == 0) {
@@ -430,7 +430,8 @@ bool conv3_big_ok(const GemmArgs& g) {
 
 bool conv3_big_stats_ok(const GemmArgs& g) {
   const uint64_t hw = (uint64_t)g.Ho * g.Wo;
-  return hw % 64 == 0 && (uint64_t)((g.Ho + 15) / 16) * ((g.Wo + 15) / 16) <= hw / 64;
+  return (hw % 64 == 0 || g.M == hw) &&
+         (uint64_t)((g.Ho + 15) / 16) * ((g.Wo + 15) / 16) <= (hw + 63) / 64;
 }
 
 uint32_t conv3_big_tiles(const GemmArgs& g) {

@@ -590,7 +590,7 @@ constexpr uint32_t kGnApplyWgs = 256;
 constexpr uint32_t kGnSideX = 2560;  // B * K floats of a side-job GEMV's input
 
 // Pre-fold of producer statistics for large images: every apply workgroup
-// otherwise re-reads all HW / 64 chunks of its channel slice (2 MB per
+// otherwise re-reads all ceil(HW / 64) chunks of its channel slice (2 MB per
 // workgroup at 512 x 512).  out[n][k][c][2] = sum over chunks
 // [k * F, min((k + 1) * F, cpi)) of st[n][chunk][c][2]; one thread per
 // (channel, statistic) pair, consecutive threads on consecutive floats.
@@ -619,7 +619,7 @@ __global__ __launch_bounds__(256) void k_gn_stats_fold(GnStats st, float* __rest
       ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
 }
 
-// cpi: statistics chunks per image in st (HW / 64 as the GEMM epilogue wrote
+// cpi: statistics chunks per image in st (ceil(HW / 64) as the GEMM epilogue wrote
 // them, or fewer after k_gn_stats_fold).
 // NU: statistics chunks each lane loads in the first, straight-line batch
 // (the host picks the smallest of 1 / 2 / 4 / 8 that covers the image's
@@ -1267,8 +1267,8 @@ void launch_group_norm_nhwc(hipStream_t s, NhwcSrc x, const float* gamma, const 
   }
 }
 
-bool gn_stats_slice(uint32_t C, uint32_t G, uint32_t HW, uint32_t* sw) {
-  if (G == 0 || C % G != 0 || HW % 64 != 0) return false;
+bool gn_stats_slice(uint32_t C, uint32_t G, uint32_t* sw) {
+  if (G == 0 || C % G != 0) return false;
   const uint32_t cpg = C / G;
   uint32_t l = cpg;
   while (l % 8 != 0) l += cpg;  // lcm(cpg, 8)
@@ -1282,7 +1282,7 @@ bool gn_stats_slice(uint32_t C, uint32_t G, uint32_t HW, uint32_t* sw) {
 }
 
 uint64_t gn_fold_ws_floats(uint32_t N, uint32_t C, uint32_t HW) {
-  const uint32_t cpi = HW / 64;
+  const uint32_t cpi = (HW + 63) / 64;
   if (cpi <= kGnFoldMin) return 0;
   const uint32_t F = (cpi + kGnFoldTarget - 1) / kGnFoldTarget;
   return (uint64_t)N * ((cpi + F - 1) / F) * C * 2;
@@ -1298,10 +1298,11 @@ bool launch_group_norm_nhwc_st(hipStream_t s, NhwcSrc x, const GnStats& st_in, c
                                uint32_t HW, float eps, bool silu, float* fold_ws,
                                const GemvArgs* side) {
   uint32_t sw = 0;
-  if (!gn_stats_slice(C, G, HW, &sw) || x.c1 % 8 != 0 || (st_in.c1 < C && st_in.c1 % 8 != 0))
+  if (!gn_stats_chunks_ok(N, HW) || !gn_stats_slice(C, G, &sw) || x.c1 % 8 != 0 ||
+      (st_in.c1 < C && st_in.c1 % 8 != 0))
     return false;
   GnStats st = st_in;
-  uint32_t cpi = HW / 64;
+  uint32_t cpi = (HW + 63) / 64;
   if (fold_ws && cpi > kGnFoldMin) {
     const uint32_t F = (cpi + kGnFoldTarget - 1) / kGnFoldTarget, cpo = (cpi + F - 1) / F;
     k_gn_stats_fold<<<dim3((2 * C + 255) / 256, cpo, N), 256, 0, s>>>(st_in, fold_ws, C, cpi, F,

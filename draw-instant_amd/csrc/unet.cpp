@@ -438,7 +438,7 @@ int unet_step(Ctx* c, UNet& u, const float* sample, const float* tsteps, const f
     launch_gemv(g3, DI_F16, c->stream);
   }
 
-  // An activation and, when its level allows (HW % 64 == 0), the GroupNorm
+  // An activation and, when its level allows (gn_stats_chunks_ok), the GroupNorm
   // statistics its producer wrote (every GN input here is the output of a
   // GEMM epilogue, so no GN runs a separate statistics pass).
   struct Act {
@@ -452,7 +452,7 @@ int unet_step(Ctx* c, UNet& u, const float* sample, const float* tsteps, const f
     a.c = ch;
     a.has_st = false;
     int r = a.buf.alloc(c, rows * ch * 2);
-    if (!r && (hh * ww) % 64 == 0) r = a.st.alloc(c, gn_stats_floats(rows, ch) * sizeof(float));
+    if (!r && gn_stats_chunks_ok(B, hh * ww)) r = a.st.alloc(c, gn_stats_floats(rows, ch) * sizeof(float));
     a.so = StatsOut{a.st.f(), false};
     return r;
   };

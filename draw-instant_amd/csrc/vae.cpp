@@ -223,7 +223,7 @@ int vae_decode_step(Ctx* c, Vae& v, const float* z, float* img, uint32_t B, uint
   const uint32_t G = cf.groups;
   const uint32_t L = cf.latent_channels, lp = (L + 7) / 8 * 8;
 
-  // an activation and (HW % 64 == 0) the GroupNorm statistics its producer wrote
+  // an activation and (gn_stats_chunks_ok) the GroupNorm statistics its producer wrote
   struct Act {
     Scratch buf, st;
     uint32_t c = 0;
@@ -235,7 +235,7 @@ int vae_decode_step(Ctx* c, Vae& v, const float* z, float* img, uint32_t B, uint
     a.c = ch;
     a.has_st = false;
     int r = a.buf.alloc(c, rows * ch * 2);
-    if (!r && (hh * ww) % 64 == 0) r = a.st.alloc(c, gn_stats_floats(rows, ch) * sizeof(float));
+    if (!r && gn_stats_chunks_ok(B, hh * ww)) r = a.st.alloc(c, gn_stats_floats(rows, ch) * sizeof(float));
     a.so = StatsOut{a.st.f(), false};
     return r;
   };
