@@ -28,6 +28,8 @@ struct AttnArgs {
   // key groups inside a workgroup (1 or 2; set by run_attention, only
   // without a split): see k_flash_attn
   uint32_t key_groups = 1;
+  // 16-query groups per wave (1 or 2; set by run_attention)
+  uint32_t query_groups = 1;
   // fp32 tensors: q32 / o32 (strides as q / o, in elements) take the place of
   // q / o, and k32 / v32 of k / v; null: the fp16 pointers
   const float* q32 = nullptr;

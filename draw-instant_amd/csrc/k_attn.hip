@@ -122,12 +122,18 @@ __device__ __forceinline__ float sum_q4(float x) {
 // single-group kernel (which may be split over workgroups and merged by
 // k_attn_combine).
 //
+// QG (1 or 2) groups of 16 queries per wave: with two every K and V fragment
+// read from LDS feeds two MFMAs (64 KiB of reads for 64 x 64 scores are 512
+// clocks of a CU's LDS, their MFMAs 256), for 133 registers instead of 88:
+// three workgroups of 128 queries per CU instead of four of 64
+// (attn_query_groups).
+//
 // IO: 0 = fp16 tensors; 1 = fp32 queries and outputs (rounded to fp16 as the
 // query fragments are built, stored unrounded); 2 = fp32 keys and values too,
 // which then go through registers into the same LDS image: the next tile's
 // loads are issued at the start of a tile and rounded and stored at its end.
-template <int KS, int IO>
-__global__ __launch_bounds__(256 * KS, 4) void k_flash_attn(AttnArgs a, uint32_t nqb) {
+template <int KS, int IO, int QG>
+__global__ __launch_bounds__(256 * KS, QG == 1 ? 4 : 3) void k_flash_attn(AttnArgs a, uint32_t nqb) {
   __shared__ __attribute__((aligned(16))) unsigned char smem[KS * 2 * BUF_BYTES];  // [kg][buf][K | V]
   kernarg_warm(a);
 
@@ -151,10 +157,12 @@ __global__ __launch_bounds__(256 * KS, 4) void k_flash_attn(AttnArgs a, uint32_t
   const uint64_t oo = b * a.bo + h * a.ho;
 
   // Q'^T fragments for the two 32-wide d steps
-  const uint32_t qrow = qb * 64 + wave * 16 + r;
-  f16x8 qf[2];
+  const uint32_t qrow0 = qb * (64 * QG) + wave * (16 * QG) + r;
+  f16x8 qf[QG][2];
 #pragma unroll
-  for (int ks = 0; ks < 2; ks++) {
+  for (int i = 0; i < 2 * QG; i++) {
+    const int qi = i / 2, ks = i % 2;
+    const uint32_t qrow = qrow0 + qi * 16;
     f16x8 t = {};
     if (qrow < a.Sq) {
       const uint64_t at = qo + (uint64_t)qrow * a.ldq + ks * 32 + g * 8;
@@ -170,7 +178,7 @@ __global__ __launch_bounds__(256 * KS, 4) void k_flash_attn(AttnArgs a, uint32_t
       }
     }
 #pragma unroll
-    for (int j = 0; j < 8; j++) qf[ks][j] = (f16)((float)t[j] * a.scale_log2);
+    for (int j = 0; j < 8; j++) qf[qi][ks][j] = (f16)((float)t[j] * a.scale_log2);
   }
 
   // K / V tiles straight into LDS: wave w moves rows 16w .. 16w+15 of each,
@@ -226,11 +234,16 @@ __global__ __launch_bounds__(256 * KS, 4) void k_flash_attn(AttnArgs a, uint32_t
     }
   };
 
-  float m = 0.0f, l = 0.0f;  // running max (log2 units) and this lane's partial row sum
-  f32x4 negm = {0.f, 0.f, 0.f, 0.f};  // -m: the score MFMAs' accumulator start
-  f32x4 o[4];
+  float m[QG], l[QG];  // running max (log2 units) and this lane's partial row sum
+  f32x4 negm[QG];      // -m: the score MFMAs' accumulator start
+  f32x4 o[QG][4];
 #pragma unroll
-  for (int dt = 0; dt < 4; dt++) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int qi = 0; qi < QG; qi++) {
+    m[qi] = l[qi] = 0.0f;
+    negm[qi] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int dt = 0; dt < 4; dt++) o[qi][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
 
   // K fragment (kt, ks): row kt*16 + r, chunk 4ks + g
   const uint32_t k_rd0 = k_off(r, g), k_rd1 = k_off(r, 4 + g);
@@ -262,63 +275,73 @@ __global__ __launch_bounds__(256 * KS, 4) void k_flash_attn(AttnArgs a, uint32_t
     if (t + 1 < t1) dma_kv(t + 1, Int<cur ^ 1>{});
 
     // S' = K Q'^T - m
-    f32x4 s[4];
+    f32x4 s[QG][4];
 #pragma unroll
     for (int kt = 0; kt < 4; kt++) {
       const f16x8 k0 = *(const f16x8*)(sb + k_rd0 + kt * 2048);
       const f16x8 k1 = *(const f16x8*)(sb + k_rd1 + kt * 2048);
-      s[kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k0, qf[0], negm, 0, 0, 0);
-      s[kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k1, qf[1], s[kt], 0, 0, 0);
+#pragma unroll
+      for (int qi = 0; qi < QG; qi++) {
+        s[qi][kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k0, qf[qi][0], negm[qi], 0, 0, 0);
+        s[qi][kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k1, qf[qi][1], s[qi][kt], 0, 0, 0);
+      }
     }
     if ((uint32_t)(t + 1) * BKV > a.Skv) {
 #pragma unroll
       for (int kt = 0; kt < 4; kt++)
 #pragma unroll
         for (int i = 0; i < 4; i++)
-          if ((uint32_t)(t * BKV + kt * 16 + 4 * g + i) >= a.Skv) s[kt][i] = -INFINITY;
+          if ((uint32_t)(t * BKV + kt * 16 + 4 * g + i) >= a.Skv) {
+#pragma unroll
+            for (int qi = 0; qi < QG; qi++) s[qi][kt][i] = -INFINITY;
+          }
     }
     // raise the running max by this tile's excess over it (>= 0 after the
     // first tile; on the first, o and l are still zero)
-    auto raise_max = [&](bool first) {
-      float mx = fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3]));
+    auto raise_max = [&](int qi, bool first) {
+      float mx = fmaxf(fmaxf(s[qi][0][0], s[qi][0][1]), fmaxf(s[qi][0][2], s[qi][0][3]));
 #pragma unroll
       for (int kt = 1; kt < 4; kt++)
-        mx = fmaxf(fmaxf(mx, fmaxf(s[kt][0], s[kt][1])), fmaxf(s[kt][2], s[kt][3]));
+        mx = fmaxf(fmaxf(mx, fmaxf(s[qi][kt][0], s[qi][kt][1])),
+                   fmaxf(s[qi][kt][2], s[qi][kt][3]));
       mx = max_q4(mx);
       const float dl = first ? mx : fmaxf(mx, 0.0f);
-      m += dl;
-      negm -= dl;
+      m[qi] += dl;
+      negm[qi] -= dl;
 #pragma unroll
-      for (int kt = 0; kt < 4; kt++) s[kt] -= dl;
+      for (int kt = 0; kt < 4; kt++) s[qi][kt] -= dl;
       const float alpha = first ? 0.0f : __builtin_amdgcn_exp2f(-dl);
-      l *= alpha;
+      l[qi] *= alpha;
 #pragma unroll
-      for (int dt = 0; dt < 4; dt++) o[dt] *= alpha;
+      for (int dt = 0; dt < 4; dt++) o[qi][dt] *= alpha;
     };
-    if (t == t0) raise_max(true);
-    f16x8 pf[2];
-    float ts;
-    auto probs = [&]() {
-      ts = 0.0f;
+    f16x8 pf[QG][2];
+    float ts[QG];
+    auto probs = [&](int qi) {
+      ts[qi] = 0.0f;
 #pragma unroll
       for (int kt = 0; kt < 4; kt++)
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-          const float p = __builtin_amdgcn_exp2f(s[kt][i]);
-          ts += p;
-          pf[kt >> 1][(kt & 1) * 4 + i] = (f16)p;
+          const float p = __builtin_amdgcn_exp2f(s[qi][kt][i]);
+          ts[qi] += p;
+          pf[qi][kt >> 1][(kt & 1) * 4 + i] = (f16)p;
         }
     };
-    probs();
-    // a probability above kLaneSumMax (or inf / NaN from an overflowing
-    // score) shows in its lane's sum: rescale and redo the tile.  The test
-    // compares the sum's bits as an integer (sign cleared), which orders
-    // finite < inf < NaN and which -fno-honor-nans cannot fold away.
-    if (__builtin_amdgcn_ballot_w64((__float_as_uint(ts) & 0x7fffffffu) > kLaneSumMaxBits) != 0) {
-      raise_max(false);
-      probs();
+#pragma unroll
+    for (int qi = 0; qi < QG; qi++) {
+      if (t == t0) raise_max(qi, true);
+      probs(qi);
+      // a probability above kLaneSumMax (or inf / NaN from an overflowing
+      // score) shows in its lane's sum: rescale and redo the tile.  The test
+      // compares the sum's bits as an integer (sign cleared), which orders
+      // finite < inf < NaN and which -fno-honor-nans cannot fold away.
+      if (__builtin_amdgcn_ballot_w64((__float_as_uint(ts[qi]) & 0x7fffffffu) > kLaneSumMaxBits) != 0) {
+        raise_max(qi, false);
+        probs(qi);
+      }
+      l[qi] += ts[qi];
     }
-    l += ts;
     // O^T += V^T P^T over two 32-key k steps
 #pragma unroll
     for (int ks = 0; ks < 2; ks++) {
@@ -328,7 +351,9 @@ __global__ __launch_bounds__(256 * KS, 4) void k_flash_attn(AttnArgs a, uint32_t
         const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)vp);
         const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(vp + 16 * 128));
         const f16x8 vf = __builtin_bit_cast(f16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-        o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pf[ks], o[dt], 0, 0, 0);
+#pragma unroll
+        for (int qi = 0; qi < QG; qi++)
+          o[qi][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pf[qi][ks], o[qi][dt], 0, 0, 0);
       }
     }
     // the next tile has landed in LDS (vmcnt 0), every wave is done with this one
@@ -351,8 +376,10 @@ __global__ __launch_bounds__(256 * KS, 4) void k_flash_attn(AttnArgs a, uint32_t
     tile(Int<0>{}, t0 + i);
     if (i + 1 < tpg) tile(Int<1>{}, t0 + i + 1);
   }
-  l = sum_q4(l);
+#pragma unroll
+  for (int qi = 0; qi < QG; qi++) l[qi] = sum_q4(l[qi]);
   if constexpr (KS > 1) {
+    static_assert(KS == 1 || QG == 1, "key groups with one query group");
     // merge the key groups: groups 1..KS-1 leave (m, row sum, unnormalised
     // O) in LDS, lane by lane (float j of lane l at [slot][j][l]); group 0
     // rescales every part to the largest max and adds them.  The K / V
@@ -365,16 +392,16 @@ __global__ __launch_bounds__(256 * KS, 4) void k_flash_attn(AttnArgs a, uint32_t
 #pragma unroll
       for (int dt = 0; dt < 4; dt++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) dst[(dt * 4 + i) * 64] = o[dt][i];
-      dst[16 * 64] = m;
-      dst[17 * 64] = l;
+        for (int i = 0; i < 4; i++) dst[(dt * 4 + i) * 64] = o[0][dt][i];
+      dst[16 * 64] = m[0];
+      dst[17 * 64] = l[0];
     }
     __syncthreads();
     if (kg > 0) return;
     float ms[KS], ls[KS];
-    ms[0] = m;
-    ls[0] = l;
-    float mx = m;
+    ms[0] = m[0];
+    ls[0] = l[0];
+    float mx = m[0];
 #pragma unroll
     for (int k = 1; k < KS; k++) {
       const float* src = xs + ((k - 1) * 4 + wave) * NF * 64 + lane;
@@ -382,28 +409,31 @@ __global__ __launch_bounds__(256 * KS, 4) void k_flash_attn(AttnArgs a, uint32_t
       ls[k] = src[17 * 64];
       mx = fmaxf(mx, ms[k]);
     }
-    float wk = __builtin_amdgcn_exp2f(m - mx);
-    l = ls[0] * wk;
+    float wk = __builtin_amdgcn_exp2f(m[0] - mx);
+    l[0] = ls[0] * wk;
 #pragma unroll
-    for (int dt = 0; dt < 4; dt++) o[dt] *= wk;
+    for (int dt = 0; dt < 4; dt++) o[0][dt] *= wk;
 #pragma unroll
     for (int k = 1; k < KS; k++) {
       const float* src = xs + ((k - 1) * 4 + wave) * NF * 64 + lane;
       wk = __builtin_amdgcn_exp2f(ms[k] - mx);
-      l += ls[k] * wk;
+      l[0] += ls[k] * wk;
 #pragma unroll
       for (int dt = 0; dt < 4; dt++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) o[dt][i] += src[(dt * 4 + i) * 64] * wk;
+        for (int i = 0; i < 4; i++) o[0][dt][i] += src[(dt * 4 + i) * 64] * wk;
     }
   }
-  if (qrow < a.Sq) {
-    const float inv = 1.0f / l;
+#pragma unroll
+  for (int qi = 0; qi < QG; qi++) {
+    const uint32_t qrow = qrow0 + qi * 16;
+    if (qrow >= a.Sq) break;
+    const float inv = 1.0f / l[qi];
     if (IO > 0 && a.splits == 1) {
       float* d32 = a.o32 + oo + (uint64_t)qrow * a.ldo;
 #pragma unroll
-      for (int dt = 0; dt < 4; dt++) *(f32x4*)(d32 + dt * 16 + g * 4) = o[dt] * inv;
-      return;
+      for (int dt = 0; dt < 4; dt++) *(f32x4*)(d32 + dt * 16 + g * 4) = o[qi][dt] * inv;
+      continue;
     }
     f16* dst = IO > 0 ? nullptr : a.o + oo + (uint64_t)qrow * a.ldo;
     if (a.splits > 1) {
@@ -411,13 +441,13 @@ __global__ __launch_bounds__(256 * KS, 4) void k_flash_attn(AttnArgs a, uint32_t
       // (b, h, q) of the [splits][B*H*Sq] workspace
       const uint64_t prow = ((uint64_t)split * a.rows + (uint64_t)hb * a.Sq + qrow);
       dst = a.part_o + prow * D;
-      if (g == 0) *(float2*)(a.part_ml + prow * 2) = float2{m, l};
+      if (g == 0) *(float2*)(a.part_ml + prow * 2) = float2{m[qi], l[qi]};
     }
 #pragma unroll
     for (int dt = 0; dt < 4; dt++) {
       f16x4 ov;
 #pragma unroll
-      for (int i = 0; i < 4; i++) ov[i] = (f16)(o[dt][i] * inv);
+      for (int i = 0; i < 4; i++) ov[i] = (f16)(o[qi][dt][i] * inv);
       *(f16x4*)(dst + dt * 16 + g * 4) = ov;
     }
   }
@@ -508,12 +538,43 @@ uint32_t attn_key_groups(const Ctx* c, uint32_t B, uint32_t H, uint32_t Sq, uint
   return ks;
 }
 
+uint32_t attn_query_groups(const Ctx* c, uint32_t B, uint32_t H, uint32_t Sq, uint32_t Skv,
+                           uint32_t splits) {
+  // Two query groups a wave where 64-query workgroups about fill the chip (four
+  // a CU) or more and each walks 20 or more key tiles, 32 or more where the
+  // 128-query ones (three a CU) need a second round.  Measured at the same split
+  // count, bit-identical: 1440 workgroups (2 x 5 heads x 9216 queries and keys)
+  // 262 -> 222 us, 2560 (8 x 5 x 4096) 199 -> 172, 960 (3 x 5 x 4096) 80.3 ->
+  // 72.7, in three ranges (1 x 5 x 4096) 35.3 -> 33.7.  Half as many workgroups
+  // leave CUs short of waves below that (752: 48.9 -> 52.1, 640: 61 -> 67); a
+  // short second round costs more than it gains (1680 of 21 tiles: 49.9 -> 51.8),
+  // and with 16 tiles or the 2 of cross-attention the two are even.
+  const uint64_t blocks = (uint64_t)((Sq + 63) / 64) * H * B * splits;
+  const uint32_t n = (Skv + BKV - 1) / BKV / splits, cus = (uint32_t)c->num_cus;
+  uint32_t qg = blocks * 10 >= 36ull * cus && n >= (blocks <= 6ull * cus ? 20u : 32u) ? 2u : 1u;
+  // tuning override: DI_ATTN_QGROUPS=1|2, read per call
+  if (const char* env = getenv("DI_ATTN_QGROUPS")) {
+    const uint32_t want = (uint32_t)atoi(env);
+    if (want == 1 || want == 2) qg = want;
+  }
+  return qg;
+}
+
 template <int IO>
 static void launch_flash(const AttnArgs& a, uint32_t B, hipStream_t s) {
-  const uint32_t nqb = (a.Sq + 63) / 64;
-  const dim3 grid(nqb * a.H * B * a.splits);
-  if (a.splits == 1 && a.key_groups == 2) k_flash_attn<2, IO><<<grid, 512, 0, s>>>(a, nqb);
-  else k_flash_attn<1, IO><<<grid, 256, 0, s>>>(a, nqb);
+  const uint32_t nqb = (a.Sq + 63) / 64, nqb2 = (a.Sq + 127) / 128;
+  const dim3 grid(nqb * a.H * B * a.splits), grid2(nqb2 * a.H * B * a.splits);
+  if (a.splits == 1 && a.key_groups == 2) {
+    k_flash_attn<2, IO, 1><<<grid, 512, 0, s>>>(a, nqb);
+    return;
+  }
+  if constexpr (IO < 2) {
+    if (a.query_groups == 2) {
+      k_flash_attn<1, IO, 2><<<grid2, 256, 0, s>>>(a, nqb2);
+      return;
+    }
+  }
+  k_flash_attn<1, IO, 1><<<grid, 256, 0, s>>>(a, nqb);
 }
 
 template <bool F32>
@@ -557,6 +618,7 @@ int run_attention(Ctx* c, AttnArgs a, uint32_t B) {
     a.splits = (n_tiles + tps - 1) / tps;
   }
   a.key_groups = attn_key_groups(c, B, a.H, a.Sq, a.Skv, a.splits);
+  a.query_groups = attn_query_groups(c, B, a.H, a.Sq, a.Skv, a.splits);
   a.rows = (uint64_t)B * a.H * a.Sq;
   void* ws = nullptr;
   uint64_t cap = 0;
