@@ -70,7 +70,12 @@ int run(Ctx* c, GemmArgs& g, int a_mode, StatsOut* st = nullptr, RowStatsOut* rs
   if (g.splits > 1 || g.part_only) {
     void* ws = nullptr;
     int rc = workspace(c, gemm_ws_bytes(g), &ws);
-    if (rc) return rc;
+    if (rc && (g.part_only || g.part_slots || (gn && gn->done))) return rc;
+    if (rc) {
+      // no memory for the partials: the problem also runs in one piece
+      (void)hipGetLastError();
+      g.splits = 1;
+    }
     g.part = (float*)ws;
   }
   if (gn && gn->done) g.part_cpg = g.N / gn->f.groups;

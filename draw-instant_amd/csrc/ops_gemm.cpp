@@ -16,12 +16,10 @@ int run_gemm(di_ctx* ctx, GemmArgs& g, int elem, int a_mode, int b_mode, int til
   if (g.splits > 1) {
     void* ws = nullptr;
     int rc = workspace(ctx, gemm_ws_bytes(g), &ws);
-    if (rc && elem == DI_F32) {
-      // no memory for the partials: fp32 problems also run in one piece
+    if (rc) {
+      // no memory for the partials: the problem also runs in one piece
       (void)hipGetLastError();
       g.splits = 1;
-    } else if (rc) {
-      return rc;
     }
     g.part = (float*)ws;
   }
