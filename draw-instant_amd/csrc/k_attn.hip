@@ -540,18 +540,18 @@ uint32_t attn_key_groups(const Ctx* c, uint32_t B, uint32_t H, uint32_t Sq, uint
 
 uint32_t attn_query_groups(const Ctx* c, uint32_t B, uint32_t H, uint32_t Sq, uint32_t Skv,
                            uint32_t splits) {
-  // Two query groups a wave where 64-query workgroups about fill the chip (four
-  // a CU) or more and each walks 20 or more key tiles, 32 or more where the
+  // Two query groups a wave where 64-query workgroups come to more than three a
+  // CU and each walks 20 or more key tiles, 32 or more where the
   // 128-query ones (three a CU) need a second round.  Measured at the same split
   // count, bit-identical: 1440 workgroups (2 x 5 heads x 9216 queries and keys)
   // 262 -> 222 us, 2560 (8 x 5 x 4096) 199 -> 172, 960 (3 x 5 x 4096) 80.3 ->
-  // 72.7, in three ranges (1 x 5 x 4096) 35.3 -> 33.7.  Half as many workgroups
-  // leave CUs short of waves below that (752: 48.9 -> 52.1, 640: 61 -> 67); a
+  // 72.7, in three ranges (1 x 5 x 4096) 35.3 -> 33.7, 832 (1 x 13 x 4096) 80.0 ->
+  // 72.8.  Half as many workgroups leave CUs short of waves below that (752: 48.9 -> 52.1, 640: 61 -> 67); a
   // short second round costs more than it gains (1680 of 21 tiles: 49.9 -> 51.8),
   // and with 16 tiles or the 2 of cross-attention the two are even.
   const uint64_t blocks = (uint64_t)((Sq + 63) / 64) * H * B * splits;
   const uint32_t n = (Skv + BKV - 1) / BKV / splits, cus = (uint32_t)c->num_cus;
-  uint32_t qg = blocks * 10 >= 36ull * cus && n >= (blocks <= 6ull * cus ? 20u : 32u) ? 2u : 1u;
+  uint32_t qg = blocks * 10 >= 32ull * cus && n >= (blocks <= 6ull * cus ? 20u : 32u) ? 2u : 1u;
   // tuning override: DI_ATTN_QGROUPS=1|2, read per call
   if (const char* env = getenv("DI_ATTN_QGROUPS")) {
     const uint32_t want = (uint32_t)atoi(env);
