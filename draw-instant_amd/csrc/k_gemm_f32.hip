@@ -2,18 +2,21 @@
 // for the executor's fp32 ops (matmul wgsl-ops.js:477-556, gemm :821-897, convMM
 // :584-698) and the fp32 linears.
 //
-// Every fp32 operand value is split, as its tile is staged, into three bf16
-// parts x = h + m + l (each the rounding of what the parts before it left, so
-// the sum is exact), and a product is the six MFMA products of parts whose
+// Every fp32 operand value is scaled by 2^16 and split, as its tile is staged,
+// into three bf16 parts x = h + m + l (each the rounding of what the parts
+// before it left; bf16 reaches down to 2^-133, the scaled value's last bit to
+// 2^-133 or above, so the sum is exact, subnormals included; the method is
+// Henry, Tang and Heinecke's, ARITH 2019), and a product is the six MFMA products of parts whose
 // weight is above 2^-24: h h, h m, m h, m m, h l, l h.  The three products
 // left out are below the rounding of one fp32 product.  The matrix cores do
 // bf16 at 16 times the fp32 MFMA rate, so six products still leave 2.7 times
 // the fp32 MFMA's peak, and one bf16 MFMA sums 32 products where the fp32 one
-// sums 4: fewer roundings of the running sum, a smaller error.
+// sums 4: fewer roundings of the running sum, a smaller error.  The sums are
+// scaled back, exactly, before the epilogue.
 //
-// Infinities and NaNs have no such split (inf - inf).  They, and a finite
-// value that rounds up to a bf16 infinity, leave a non-finite sum in every
-// output they reach; a workgroup that finds one in its tile computes the tile
+// Infinities and NaNs have no such split (inf - inf).  They, and values and
+// sums that overflow scaled (from 2^112 and 2^96 on), leave a non-finite sum in
+// every output they reach; a workgroup that finds one in its tile computes the tile
 // again with the fp32 MFMA on the unsplit values, so those results are the
 // fp32 instruction's own.
 //
@@ -24,8 +27,12 @@
 // work, a PFLOP/s of bf16; the fp32 MFMA's peak is 157), batched 5 x 2304 x
 // 2304 x 64 90 -> 53 us.  Error against 64 bits (relative 2-norm): 1.4e-6 ->
 // 2.5e-7, 8.0e-7 -> 4.9e-7 over both linears, and between 0.3 and 0.9 times the
-// old kernel's on every shape tried.  What bounds it is the split-and-store
-// phase (5.5 VALU operations per staged value) that one workgroup's MFMAs hide
+// old kernel's on every shape tried.  The times are those before the scaling,
+// which costs 1 to 3 % (2048 x 5120 x 1280 168.1 -> 171.5 us, 2048 x 1280 x 5120
+// 154.4 -> 157.5, 512 -> 512 at 64 x 64 113.7 -> 117.0 in turn on one card) and
+// without which operands below 2^-110 lost bits: a relative error of 1e-6 at
+// 2^-116, 2e-3 at 2^-126 and 1 at 2^-135, now 1e-7 throughout.  What bounds it is the split-and-store
+// phase (6.5 VALU operations per staged fp32 value) that one workgroup's MFMAs hide
 // from another only in part.
 #include <cstdlib>
 #include <type_traits>
@@ -45,8 +52,17 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr uint32_t kOut = 0x80000000u;  // a buffer offset past every extent: reads 0
 
-// Two fp32 values -> their h, m and l parts, each a packed bf16 pair.
+// fp32 operands are split times 2^16: the last bit of the smallest subnormal,
+// 2^-149, is then bf16's own smallest step, 2^-133, and every part of every
+// fp32 value is held.  (fp16-resident B: two parts hold a value of any size.)
+template <typename T>
+constexpr float kScale = sizeof(T) == 4 ? 0x1p16f : 1.0f;
+
+// Two values of a T operand, scaled -> their h, m and l parts, each a packed bf16 pair.
+template <typename T>
 __device__ __forceinline__ void split2(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
+  a *= kScale<T>;
+  b *= kScale<T>;
   h = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
   const float ra = a - __uint_as_float(h << 16), rb = b - __uint_as_float(h & 0xffff0000u);
   m = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{ra, rb}, bf16x2));
@@ -76,7 +92,7 @@ __device__ __forceinline__ uint32_t plane_at(uint32_t row, uint32_t c) {
   return row * 64 + ((c ^ ((row >> 2) & 3)) << 4);
 }
 
-template <int ROWS>
+template <typename T, int ROWS>
 __device__ __forceinline__ void store_split(char* s, const F32Tile<ROWS>& t, bool kmajor) {
   constexpr uint32_t P = ROWS * 64;  // bytes of one plane
   const uint32_t tid = threadIdx.x;
@@ -89,7 +105,7 @@ __device__ __forceinline__ void store_split(char* s, const F32Tile<ROWS>& t, boo
 #pragma unroll
       for (int j = 0; j < 2; j++) {
         uint32_t a, b, c;
-        split2(t.v[4 * i + 2 * j], t.v[4 * i + 2 * j + 1], a, b, c);
+        split2<T>(t.v[4 * i + 2 * j], t.v[4 * i + 2 * j + 1], a, b, c);
         h[j] = a;
         m[j] = b;
         l[j] = c;
@@ -107,7 +123,7 @@ __device__ __forceinline__ void store_split(char* s, const F32Tile<ROWS>& t, boo
 #pragma unroll
       for (int j = 0; j < 4; j++) {
         uint32_t a, b, c;
-        split2(t.v[8 * i + 2 * j], t.v[8 * i + 2 * j + 1], a, b, c);
+        split2<T>(t.v[8 * i + 2 * j], t.v[8 * i + 2 * j + 1], a, b, c);
         h[j] = a;
         m[j] = b;
         l[j] = c;
@@ -396,8 +412,8 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f32(GemmArgs g) {
       LB.load(k_begin, tb);
     }
     for (uint32_t s = 0; s < n_stages; s++) {
-      store_split(sA, ta, A_KMAJ);
-      store_split(sB, tb, B_KMAJ);
+      store_split<float>(sA, ta, A_KMAJ);
+      store_split<TB>(sB, tb, B_KMAJ);
       if (s + 1 < n_stages) {  // on its way while this stage is computed
         LA.load(k_begin + (s + 1) * 32, ta);
         LB.load(k_begin + (s + 1) * 32, tb);
@@ -467,6 +483,12 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f32(GemmArgs g) {
       }
     }
     __syncthreads();  // read before the strips below take the memory
+  } else {
+    constexpr float unscale = 1.0f / (kScale<float> * kScale<TB>);
+#pragma unroll
+    for (int a = 0; a < TM; a++)
+#pragma unroll
+      for (int b = 0; b < TN; b++) acc[a][b] *= unscale;
   }
 
   // ---- store ----

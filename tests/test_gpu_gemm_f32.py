@@ -126,3 +126,38 @@ def test_non_finite(dev, rng, M, N, K):
     assert np.array_equal(got[bad & ~np.isnan(ref)], ref[bad & ~np.isnan(ref)])
     rows = [i for i in range(M) if i not in (0, 2, 5)]
     _check(got[rows], ref[rows], mag[rows], K)
+
+
+# Operands down to fp32's smallest subnormals (2^-149) and up to the overflow of
+# the scaled split (2^112, sums of 2^96): every bit of either counts against a
+# partner that brings the product back to an ordinary size.
+SCALES = [(-102, 100), (-111, 100), (-118, 100), (-126, 100), (-140, 100), (-60, -50), (100, -126),
+          (111, -40), (120, -20), (48, 47), (60, 60)]
+
+
+@pytest.mark.parametrize("trans_b", [0, 1])
+@pytest.mark.parametrize("ea,eb", SCALES)
+@pytest.mark.parametrize("M,N,K", [(65, 66, 40), (130, 64, 1100)])
+def test_operand_scales(dev, rng, M, N, K, ea, eb, trans_b):
+    a = (rng.standard_normal((M, K)) * 2.0 ** ea).astype(np.float32)
+    b = (rng.standard_normal((N, K) if trans_b else (K, N)) * 2.0 ** eb).astype(np.float32)
+    y = dev.create_buffer(M * N * 4)
+    _call(dev, "di_gemm", dev.storage(a).handle, dev.storage(b).handle, 0, y.handle, M, N, K,
+          trans_b, F32)
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    b64 = b64.T if trans_b else b64
+    _check(dev.download(y).reshape(M, N), a64 @ b64, np.abs(a64) @ np.abs(b64), K, 2.0 ** -149)
+
+
+@pytest.mark.parametrize("w16", [False, True])
+@pytest.mark.parametrize("ea", [-118, -130, 114])
+def test_conv_operand_scales(dev, rng, ea, w16):
+    x = (rng.standard_normal((1, 40, 9, 8)) * 2.0 ** ea).astype(np.float32)
+    w = (rng.standard_normal((66, 40, 3, 3)) * (1.0 if w16 or ea > 0 else 2.0 ** 90)) \
+        .astype(np.float16 if w16 else np.float32)
+    y = dev.create_buffer(66 * 9 * 8 * 4)
+    _call(dev, "di_conv2d", dev.storage(x).handle, dev.storage(w).handle, 0, 0, y.handle, 1, 40, 66,
+          9, 8, 3, 1, 1, 0, F32W16 if w16 else F32, NCHW)
+    x64, w64 = (torch.from_numpy(v.astype(np.float64)) for v in (x, w))
+    z, mag = (TF.conv2d(u, v, padding=1).numpy() for u, v in ((x64, w64), (x64.abs(), w64.abs())))
+    _check(dev.download(y).reshape(z.shape), z, mag, 360, 2.0 ** -149)
