@@ -562,6 +562,19 @@ const double kTileEff[TILE_COUNT] = {0.35, 0.5, 0.5, 0.8, 0.85, 0.55, 0.35, 0.5,
                                       0.5, 0.5, 0.8, 0.35, 0.8, 0.25, 0.8};
 bool vec_epi_ok(const GemmArgs& g, int elem, int tile_cfg);
 
+// What a launch may span: fewer than 2^32 threads along x (a tile's workgroup
+// has 256, eight wavefronts 512, sixteen 1024), 65535 along z (batch * splits).
+// A batch past 65535 is refused whatever its plan.
+bool grid_x_ok(uint64_t tiles, int tile_cfg) {
+  const bool k2 = tile_cfg == TILE_64x64_K2 || tile_cfg == TILE_128x64_K2 ||
+                  tile_cfg == TILE_64x128_K2 || tile_cfg == TILE_64x32_K2;
+  const bool w16 = tile_cfg >= TILE_64x128_W16 && tile_cfg <= TILE_64x64_W16;
+  return tiles * (w16 ? 1024 : k2 ? 512 : 256) < (1ull << 32);
+}
+bool grid_z_ok(uint32_t batch, uint32_t splits) {
+  return splits == 1 || (uint64_t)batch * splits <= 65535;
+}
+
 }  // namespace
 
 namespace {
@@ -596,8 +609,8 @@ bool tuned_plan(const GemmArgs& g, GemmPlan* out) {
 
 // DI_GEMM_TILE / DI_GEMM_SPLITS (tuning runs): a value that is not a whole
 // number, names no built tile (or the halo conv for a conv it cannot take),
-// or asks for splits outside [1, 64] is ignored, so no override can index
-// the tile tables out of range.
+// or asks for splits outside [1, 64] or past the grid is ignored, so no
+// override can index the tile tables out of range or fail to launch.
 static void env_plan_override(const GemmArgs& g, int elem, const char* env_tile,
                               const char* env_split, GemmPlan* plan) {
   if (env_tile) {
@@ -614,7 +627,8 @@ static void env_plan_override(const GemmArgs& g, int elem, const char* env_tile,
   if (env_split) {
     char* end = nullptr;
     const long sp = strtol(env_split, &end, 10);
-    if (end != env_split && *end == '\0' && sp >= 1 && sp <= 64) plan->splits = (uint32_t)sp;
+    if (end != env_split && *end == '\0' && sp >= 1 && sp <= 64 && grid_z_ok(g.batch, (uint32_t)sp))
+      plan->splits = (uint32_t)sp;
   }
   if (plan->splits < 1) plan->splits = 1;
 }
@@ -640,13 +654,15 @@ static GemmPlan f32_plan(const GemmArgs& g, int num_cus) {
                                {TILE_128x64, 128, 64, 3, 1.2, 0.76},
                                {TILE_64x64, 64, 64, 4, 0.88, 0.45}};
   const uint32_t stages = (g.K + 31) / 32;
-  GemmPlan best{TILE_64x64, 1};
+  GemmPlan best{TILE_128x128, 1};
   double best_t = 1e300;
   for (const Tile& t : tiles) {
-    const uint64_t T = (uint64_t)((g.M + t.bm - 1) / t.bm) * ((g.N + t.bn - 1) / t.bn) * g.batch;
-    for (uint32_t s = 1; s <= 64 && s <= stages; s++) {
+    const uint64_t xy = (uint64_t)((g.M + t.bm - 1) / t.bm) * ((g.N + t.bn - 1) / t.bn);
+    if (!grid_x_ok(xy, t.id)) continue;
+    const uint64_t T = xy * g.batch;
+    for (uint32_t s = 1; s <= 64 && s <= stages && grid_z_ok(g.batch, s); s++) {
       const uint32_t per = (stages + s - 1) / s;
-      if (s > 1 && (per < 2 || (stages + per - 1) / per != s || T * s > 65535ull * 64)) continue;
+      if (s > 1 && (per < 2 || (stages + per - 1) / per != s)) continue;
       const uint64_t w = (T * s + num_cus - 1) / num_cus;  // workgroups of the fullest CU
       const uint64_t rem = w % t.res;
       double us = (double)per * ((double)(w - rem) * t.shared +
@@ -706,15 +722,17 @@ GemmPlan f16_plan(const GemmArgs& g, int num_cus, double* est_us = nullptr) {
                                   {TILE_64x32_K2, 0.22, 0.144, 0.5, 5.05}};
   const bool is_conv = g.Cin > 0 && g.ks > 1;
   const uint32_t stages = g.K / 64;
-  GemmPlan best{TILE_64x64, 1};
+  GemmPlan best{TILE_128x128, 1};
   double best_t = 1e300;
   for (int i = 0; i < 10; i++) {
     const TileTime& t = is_conv ? conv[i] : dense[i];
     // 16 columns to a wave: only the vector epilogue pairs GEGLU's columns
     if (t.id == TILE_64x32_K2 && g.act == ACT_GEGLU && !vec_epi_ok(g, DI_F16, t.id)) continue;
-    const uint64_t T =
-        (uint64_t)((g.M + kTileM[t.id] - 1) / kTileM[t.id]) * ((g.N + kTileN[t.id] - 1) / kTileN[t.id]) * g.batch;
-    for (uint32_t s = 1; s <= 32; s++) {
+    const uint64_t xy =
+        (uint64_t)((g.M + kTileM[t.id] - 1) / kTileM[t.id]) * ((g.N + kTileN[t.id] - 1) / kTileN[t.id]);
+    if (!grid_x_ok(xy, t.id)) continue;
+    const uint64_t T = xy * g.batch;
+    for (uint32_t s = 1; s <= 32 && grid_z_ok(g.batch, s); s++) {
       const uint32_t per = (stages + s - 1) / s;
       if (s > 1 && per < 2) break;
       if (s > 1 && (stages + per - 1) / per != s) continue;  // an empty split
@@ -744,7 +762,7 @@ GemmPlan slow_plan(const GemmArgs& g, int num_cus) {
     if (g.act == ACT_GEGLU && kTileN[tc] == 160) continue;  // GEGLU pairs need even TN
     const uint64_t mt = (g.M + kTileM[tc] - 1) / kTileM[tc], nt = (g.N + kTileN[tc] - 1) / kTileN[tc];
     const uint64_t T = mt * nt * g.batch;
-    for (uint32_t s = 1; s <= 32; s++) {
+    for (uint32_t s = 1; s <= 32 && grid_z_ok(g.batch, s); s++) {
       const uint32_t kper = ((g.K + s - 1) / s + 63) / 64 * 64;
       if (s > 1 && kper < 256) break;
       const double rounds = ceil((double)T * s / cus);

@@ -1,0 +1,71 @@
+"""Plans of the contractions (gemm_plan), computed on the host: every plan's
+launch stays within what a grid may span, at the sizes where it could pass it."""
+import os
+import shutil
+import subprocess
+
+import numpy as np
+import pytest
+
+REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(REPO, "draw-instant_amd", "csrc")
+LIB = os.path.join(REPO, "draw-instant_amd", "drawinstant")
+HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+
+# rows, columns and threads of the built tiles (TileCfg)
+TILES = {0: (64, 64, 256), 1: (128, 64, 256), 2: (64, 128, 256), 3: (128, 128, 256),
+         5: (64, 160, 256), 6: (64, 64, 512), 7: (128, 64, 512), 8: (64, 128, 512),
+         9: (64, 128, 1024), 10: (128, 64, 1024), 11: (128, 128, 1024), 12: (64, 64, 1024),
+         14: (64, 32, 512)}
+F32_TILES = (0, 1, 3)  # k_gemm_f32
+
+
+@pytest.fixture(scope="module")
+def planner(tmp_path_factory):
+    if not os.path.exists(HIPCC):
+        pytest.skip("needs hipcc")
+    exe = tmp_path_factory.mktemp("plans") / "gemm_plan_check"
+    subprocess.run([HIPCC, "--offload-arch=gfx950", "-x", "hip", "-std=c++17", "-O1", "-I", CSRC,
+                    os.path.join(REPO, "tests", "gemm_plan_check.cpp"), "-o", str(exe), "-L", LIB,
+                    "-l:libdrawinstant_hip.so", "-Wl,-rpath," + LIB], check=True, timeout=300)
+
+    def plan(problems, **env):
+        """(tile, splits) of each problem: dicts of gemm_plan_check's fields."""
+        rows = []
+        for p in problems:
+            q = dict(elem=0, b_mode=0, cus=256, batch=1, act=0, cin=0, h=0, w=0, ks=1, stride=1, up=1)
+            q.update(p)
+            rows.append(" ".join(str(int(q[k])) for k in (
+                "elem", "b_mode", "cus", "batch", "M", "N", "K", "act", "cin", "h", "w", "ks",
+                "stride", "up")))
+        r = subprocess.run([str(exe)], input="\n".join(rows) + "\n", capture_output=True, text=True,
+                           timeout=120, env={**os.environ, **env}, check=True)
+        out = [tuple(int(v) for v in ln.split()) for ln in r.stdout.splitlines()]
+        assert len(out) == len(rows)
+        return out
+    return plan
+
+
+def _check(p, tile, splits):
+    bm, bn, threads = TILES[tile]
+    tiles = -(-p["M"] // bm) * -(-p["N"] // bn)
+    assert tiles * threads < 2 ** 32, (p, tile)
+    assert splits >= 1 and (splits == 1 or p.get("batch", 1) * splits <= 65535), (p, splits)
+
+
+def test_grids(planner):
+    r = np.random.default_rng(3)
+    probs = []
+    for elem in (0, 1):
+        for b_mode in (0, 1):
+            for batch in (1, 3, 1000, 5000, 10000, 20000, 32768, 65535):
+                for m, n in ((1, 1), (1, 64), (3, 500), (128, 128)):
+                    probs += [dict(elem=elem, b_mode=b_mode, batch=batch, M=m, N=n, K=k)
+                              for k in (1, 64, 512, 1024, 4096, 65536, int(r.integers(1, 9000)))]
+    # more than 2^32 / 1024 tiles of some shapes
+    probs += [dict(elem=1, M=2 ** 24, N=4096, K=64), dict(elem=1, M=2 ** 24, N=8192, K=64),
+              dict(elem=0, M=2 ** 18, N=2 ** 18, K=32), dict(elem=0, M=2 ** 24, N=4096, K=64),
+              dict(elem=0, M=1, N=2 ** 30, K=4, b_mode=1)]
+    for env in ({}, {"DI_GEMM_SPLITS": "64"}):
+        for p, (tile, splits) in zip(probs, planner(probs, **env)):
+            _check(p, tile, splits)

@@ -161,3 +161,14 @@ def test_conv_operand_scales(dev, rng, ea, w16):
     x64, w64 = (torch.from_numpy(v.astype(np.float64)) for v in (x, w))
     z, mag = (TF.conv2d(u, v, padding=1).numpy() for u, v in ((x64, w64), (x64.abs(), w64.abs())))
     _check(dev.download(y).reshape(z.shape), z, mag, 360, 2.0 ** -149)
+
+
+@pytest.mark.parametrize("batch,K", [(10000, 512), (5000, 1024), (20000, 1024), (65535, 40)])
+def test_long_batches(dev, rng, batch, K):
+    """Batches whose splits would pass the grid's 65535 along z."""
+    a, b = _mats(rng, (batch, 1, K), (batch, K, 1))
+    y = dev.create_buffer(batch * 4)
+    _call(dev, "di_matmul", dev.storage(a).handle, dev.storage(b).handle, y.handle, 1, 1, K, batch,
+          1, F32)
+    a64, b64 = a.astype(np.float64)[:, 0], b.astype(np.float64)[..., 0]
+    _check(dev.download(y).reshape(batch), (a64 * b64).sum(1), np.abs(a64 * b64).sum(1), K)
