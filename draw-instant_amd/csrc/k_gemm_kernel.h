@@ -1216,12 +1216,18 @@ void launch_cfg(const GemmArgs& g, hipStream_t s) {
       <<<dim3(tiles, 1, g.batch * g.splits), 64 * WGM * WGN * KS, 0, s>>>(g);
 }
 
-// Generic (bounds-checked) variants: two tile shapes, one for fp32 (operands
-// past the split kernel's 31-bit offsets).
+// Generic (bounds-checked) variants: two tile shapes.  fp32 (operands past the
+// split kernel's 31-bit offsets) takes the larger one only where 64 x 64 tiles
+// would pass the grid's 2^32 threads (128 -> 3 channels at 1536 x 1536: 6.8 ms on
+// 64 x 64, 16.1 on 128 x 128; 128 -> 128 13.8 and 17.3).
 template <typename T, int AM, int BMD, typename TB = T>
 void launch_slow(const GemmArgs& g, int tile_cfg, hipStream_t s) {
   if constexpr (sizeof(T) == 4) {
-    launch_cfg<T, 64, 64, 2, 2, AM, BMD, false, 2, 1, EX_NONE, TB>(g, s);
+    const uint64_t tiles = (uint64_t)((g.M + 63) / 64) * ((g.N + 63) / 64);
+    if (tiles * 256 < (1ull << 32))
+      launch_cfg<T, 64, 64, 2, 2, AM, BMD, false, 2, 1, EX_NONE, TB>(g, s);
+    else
+      launch_cfg<T, 128, 128, 2, 2, AM, BMD, false, 2, 1, EX_NONE, TB>(g, s);
     return;
   } else if (tile_cfg == TILE_64x64 || tile_cfg == TILE_128x64 || tile_cfg == TILE_64x128 ||
       tile_cfg == TILE_64x160 || tile_cfg == TILE_64x64_K2 || tile_cfg == TILE_128x64_K2 ||

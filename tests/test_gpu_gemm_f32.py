@@ -172,3 +172,54 @@ def test_long_batches(dev, rng, batch, K):
           1, F32)
     a64, b64 = a.astype(np.float64)[:, 0], b.astype(np.float64)[..., 0]
     _check(dev.download(y).reshape(batch), (a64 * b64).sum(1), np.abs(a64 * b64).sum(1), K)
+
+
+# ---- operands past 31-bit offsets: the bounds-checked fp32 MFMA kernel ----
+@pytest.mark.parametrize("w16", [False, True])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 4200007), (3, 2, 4300000)])
+def test_long_rows(dev, rng, M, N, K, w16):
+    a, b = _mats(rng, (M, K), (N, K), w16=w16)
+    y = dev.create_buffer(M * N * 4)
+    _call(dev, "di_gemm", dev.storage(a).handle, dev.storage(b).handle, 0, y.handle, M, N, K, 1,
+          F32W16 if w16 else F32)
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    _check(dev.download(y).reshape(M, N), a64 @ b64.T, np.abs(a64) @ np.abs(b64).T, K)
+
+
+@pytest.mark.parametrize("M,N,K", [(2, 16800003, 3), (1, 2 ** 30, 2)])
+def test_wide_columns(dev, rng, M, N, K):
+    """B [K][N] with rows past 31-bit offsets, the second also past 2^32 threads
+    of 64 x 64 tiles: columns from the start, the middle and the end."""
+    a = rng.standard_normal((M, K)).astype(np.float32)
+    b, y = dev.create_buffer(K * N * 4), dev.create_buffer(M * N * 4)
+    dev.fill_normal(b, K * N, 11)
+    _call(dev, "di_matmul", dev.storage(a).handle, b.handle, y.handle, M, N, K, 1, 0, F32)
+    n, a64 = 3000, a.astype(np.float64)
+    for c in (0, N // 2 - 5, N - n):
+        cols = np.stack([dev.download(b, np.float32, (n,), (k * N + c) * 4) for k in range(K)])
+        got = np.stack([dev.download(y, np.float32, (n,), (m * N + c) * 4) for m in range(M)])
+        c64 = cols.astype(np.float64)
+        _check(got, a64 @ c64, np.abs(a64) @ np.abs(c64), K)
+    b.destroy()
+    y.destroy()
+
+
+def test_large_image_conv(dev, rng):
+    """An NCHW image of more than 2^31 bytes: rows of the output at both ends."""
+    ci, co, H, W = 70, 3, 2901, 2700
+    x, y = dev.create_buffer(ci * H * W * 4), dev.create_buffer(co * H * W * 4)
+    dev.fill_normal(x, ci * H * W, 12)
+    w = rng.standard_normal((co, ci, 3, 3)).astype(np.float32)
+    _call(dev, "di_conv2d", x.handle, dev.storage(w).handle, 0, 0, y.handle, 1, ci, co, H, W, 3, 1, 1,
+          0, F32, NCHW)
+    w64 = torch.from_numpy(w.astype(np.float64))
+    for r0 in (0, H - 4):  # four input rows, of which the outer ones have a padded neighbour
+        rows = np.stack([dev.download(x, np.float32, (4, W), ((c * H) + r0) * W * 4)
+                         for c in range(ci)]).astype(np.float64)
+        t = torch.from_numpy(rows)[None]
+        z, mag = (TF.conv2d(u, v, padding=1)[0].numpy() for u, v in ((t, w64), (t.abs(), w64.abs())))
+        sl = slice(0, 3) if r0 == 0 else slice(1, 4)
+        got = np.stack([dev.download(y, np.float32, (4, W), ((o * H) + r0) * W * 4) for o in range(co)])
+        _check(got[:, sl], z[:, sl], mag[:, sl], ci * 9)
+    x.destroy()
+    y.destroy()
