@@ -608,7 +608,8 @@ bool tuned_plan(const GemmArgs& g, GemmPlan* out) {
 }  // namespace
 
 // DI_GEMM_TILE / DI_GEMM_SPLITS (tuning runs): a value that is not a whole
-// number, names no built tile (or the halo conv for a conv it cannot take),
+// number, names no tile built for the problem (fp32 has 64 x 64, 128 x 64 and
+// 128 x 128; the conv kernels take some convolutions),
 // or asks for splits outside [1, 64] or past the grid is ignored, so no
 // override can index the tile tables out of range or fail to launch.
 static void env_plan_override(const GemmArgs& g, int elem, const char* env_tile,
@@ -618,6 +619,8 @@ static void env_plan_override(const GemmArgs& g, int elem, const char* env_tile,
     const long t = strtol(env_tile, &end, 10);
     const bool ok = end != env_tile && *end == '\0' && t >= 0 && t < TILE_COUNT &&
                     t != TILE_128x160 &&
+                    (elem != DI_F32 ||
+                     t == TILE_64x64 || t == TILE_128x64 || t == TILE_128x128) &&
                     (t != TILE_CONV3_HALO ||
                      (conv3_halo_ok(g) && vec_epi_ok(g, elem, TILE_CONV3_HALO))) &&
                     (t != TILE_CONV3_BIG ||

@@ -626,13 +626,17 @@ __global__ __launch_bounds__(256) void k_f32_reduce(GemmArgs g) {
   }
 }
 
+template <int BM, int BN, int AM, int BMD, typename TB>
+void launch_f32_tile(const GemmArgs& g, hipStream_t s) {
+  const dim3 grid(((g.M + BM - 1) / BM) * ((g.N + BN - 1) / BN), 1, g.batch * g.splits);
+  k_gemm_f32<BM, BN, AM, BMD, TB><<<grid, 256, 0, s>>>(g);
+}
+
 template <int AM, int BMD, typename TB>
 void launch_f32(const GemmArgs& g, int tile, hipStream_t s) {
-  const uint32_t bm = tile == TILE_64x64 ? 64 : 128, bn = tile == TILE_128x128 ? 128 : 64;
-  const dim3 grid(((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn), 1, g.batch * g.splits);
-  if (tile == TILE_128x128) k_gemm_f32<128, 128, AM, BMD, TB><<<grid, 256, 0, s>>>(g);
-  else if (tile == TILE_128x64) k_gemm_f32<128, 64, AM, BMD, TB><<<grid, 256, 0, s>>>(g);
-  else k_gemm_f32<64, 64, AM, BMD, TB><<<grid, 256, 0, s>>>(g);
+  if (tile == TILE_128x128) launch_f32_tile<128, 128, AM, BMD, TB>(g, s);
+  else if (tile == TILE_128x64) launch_f32_tile<128, 64, AM, BMD, TB>(g, s);
+  else launch_f32_tile<64, 64, AM, BMD, TB>(g, s);
 }
 
 }  // namespace

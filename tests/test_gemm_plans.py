@@ -69,3 +69,13 @@ def test_grids(planner):
     for env in ({}, {"DI_GEMM_SPLITS": "64"}):
         for p, (tile, splits) in zip(probs, planner(probs, **env)):
             _check(p, tile, splits)
+
+
+def test_tile_override_of_fp32(planner):
+    """An override names a tile that the fp32 kernel has, or is ignored."""
+    probs = [dict(M=m, N=n, K=k, b_mode=b) for m, n, k in ((200, 70, 40), (2048, 1280, 640), (1, 9, 5000))
+             for b in (0, 1)] + [dict(M=256, N=64, K=576, cin=64, h=16, w=16, ks=3)]
+    own = planner(probs)
+    for t in range(-1, 17):
+        got = planner(probs, DI_GEMM_TILE=str(t))
+        assert got == ([(t, s) for _, s in own] if t in F32_TILES else own), t

@@ -223,3 +223,18 @@ def test_large_image_conv(dev, rng):
         _check(got[:, sl], z[:, sl], mag[:, sl], ci * 9)
     x.destroy()
     y.destroy()
+
+
+@pytest.mark.parametrize("tile", range(16))
+def test_tile_override(dev, rng, monkeypatch, tile):
+    """Every row is written whatever tile an override names."""
+    M, N, K = 200, 70, 300
+    a, b = _mats(rng, (M, K), (N, K))
+    y = dev.create_buffer(M * N * 4)
+    dev.fill_normal(y, M * N, 3)  # stale output must be overwritten
+    monkeypatch.setenv("DI_GEMM_TILE", str(tile))
+    for splits in ("1", "3"):
+        monkeypatch.setenv("DI_GEMM_SPLITS", splits)
+        _call(dev, "di_gemm", dev.storage(a).handle, dev.storage(b).handle, 0, y.handle, M, N, K, 1, F32)
+        a64, b64 = a.astype(np.float64), b.astype(np.float64)
+        _check(dev.download(y).reshape(M, N), a64 @ b64.T, np.abs(a64) @ np.abs(b64).T, K)
