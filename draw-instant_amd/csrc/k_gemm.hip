@@ -633,7 +633,7 @@ static void env_plan_override(const GemmArgs& g, int elem, const char* env_tile,
     if (end != env_split && *end == '\0' && sp >= 1 && sp <= 64 && grid_z_ok(g.batch, (uint32_t)sp))
       plan->splits = (uint32_t)sp;
   }
-  if (plan->splits < 1) plan->splits = 1;
+  if (plan->splits < 1 || plan->tile == TILE_CONV3_BIG) plan->splits = 1;  // (which has no split-K)
 }
 
 // Plan of a split-operand fp32 problem (k_gemm_f32.hip) from what its tiles
@@ -994,13 +994,6 @@ void launch_gemm(GemmArgs g, int elem, int a_mode, int b_mode, int tile_cfg, hip
     g.a2_bytes = g.a_bytes;
     if (g.c1 == 0) g.c1 = 0xffffffffu;
   }
-  const bool trace = getenv("DI_TRACE_GEMM") != nullptr;
-  if (trace)
-    fprintf(stderr,
-            "[di_gemm] M=%u N=%u K=%u batch=%u amode=%d bmode=%d elem=%d cin=%u hw=%ux%u ks=%u "
-            "stride=%u up=%u tile=%d splits=%u act=%d fast=%d\n",
-            g.M, g.N, g.K, g.batch, a_mode, b_mode, elem, g.Cin, g.H, g.W, g.ks, g.stride, g.up,
-            tile_cfg, g.splits, g.act, (int)gemm_fast_ok(g, elem, a_mode, b_mode));
   g.vec_epi = vec_epi_ok(g, elem, tile_cfg);
   const bool fast = gemm_fast_ok(g, elem, a_mode, b_mode);
   bool halo = false;
@@ -1020,6 +1013,12 @@ void launch_gemm(GemmArgs g, int elem, int a_mode, int b_mode, int tile_cfg, hip
       g.vec_epi = vec_epi_ok(g, elem, tile_cfg);
     }
   }
+  if (getenv("DI_TRACE_GEMM"))  // the tile that runs
+    fprintf(stderr,
+            "[di_gemm] M=%u N=%u K=%u batch=%u amode=%d bmode=%d elem=%d cin=%u hw=%ux%u ks=%u "
+            "stride=%u up=%u tile=%d splits=%u act=%d fast=%d\n",
+            g.M, g.N, g.K, g.batch, a_mode, b_mode, elem, g.Cin, g.H, g.W, g.ks, g.stride, g.up,
+            tile_cfg, g.splits, g.act, (int)fast);
   if (halo) {
     launch_conv3_halo(g, s);
   } else if (big) {

@@ -79,3 +79,12 @@ def test_tile_override_of_fp32(planner):
     for t in range(-1, 17):
         got = planner(probs, DI_GEMM_TILE=str(t))
         assert got == ([(t, s) for _, s in own] if t in F32_TILES else own), t
+
+
+def test_large_conv_override_does_not_split(planner):
+    """The large-image conv kernel has no split-K: an override that names it runs
+    it, in one piece, whatever the plan it replaces or the splits asked for."""
+    probs = [dict(elem=1, M=h * w, N=co, K=9 * ci, cin=ci, h=h, w=w, ks=3)
+             for ci, co, h, w in ((576, 64, 30, 31), (64, 128, 16, 16), (1280, 1280, 8, 8))]
+    for env in ({}, {"DI_GEMM_SPLITS": "3"}):
+        assert planner(probs, DI_GEMM_TILE="15", **env) == [(15, 1)] * len(probs)
