@@ -38,6 +38,18 @@ int run(Ctx* c, GemmArgs& g, int a_mode, StatsOut* st = nullptr, RowStatsOut* rs
   g.splits = plan.splits;
   g.stats = nullptr;
   g.rstats = nullptr;
+  // before anything that depends on whether the problem splits; slots shared
+  // with another launch were reserved by the caller
+  if (g.part_slots) {
+    DI_REQUIRE(g.part_only || g.splits > 1, DI_EINVAL,
+               "shared partial slots need a plan that splits (M=%u N=%u K=%u)", g.M, g.N, g.K);
+    void* ws = nullptr;
+    const int rc = workspace(c, gemm_ws_bytes(g), &ws);
+    if (rc) return rc;
+    g.part = (float*)ws;
+  } else if (const int rc = partials_workspace(c, g)) {
+    return rc;
+  }
   if (gn) {
     gn_exchange_area(c, gn->f);
     gn->done = splitk_gn_ok(g, gn->f);
@@ -67,22 +79,7 @@ int run(Ctx* c, GemmArgs& g, int a_mode, StatsOut* st = nullptr, RowStatsOut* rs
   DI_REQUIRE(!g.ln_rows || gemm_lnfold_ok(g, DI_F16, tile), DI_EUNSUPPORTED,
              "LayerNorm fold needs the vector epilogue (M=%u N=%u K=%u tile %d)", g.M, g.N, g.K,
              tile);
-  if (g.splits > 1 || g.part_only) {
-    void* ws = nullptr;
-    int rc = workspace(c, gemm_ws_bytes(g), &ws);
-    if (rc && (g.part_only || g.part_slots || (gn && gn->done))) return rc;
-    if (rc) {
-      // no memory for the partials: the problem also runs in one piece
-      (void)hipGetLastError();
-      g.splits = 1;
-    }
-    g.part = (float*)ws;
-  }
   if (gn && gn->done) g.part_cpg = g.N / gn->f.groups;
-  if (g.splits <= 1) {
-    DI_REQUIRE(g.part_only || !g.part_slots, DI_EINVAL,
-               "shared partial slots need a plan that splits (M=%u N=%u K=%u)", g.M, g.N, g.K);
-  }
   launch_gemm(g, DI_F16, a_mode, B_NK, tile, c->stream, gn && gn->done ? &gn->f : nullptr);
   return DI_OK;
 }
@@ -315,8 +312,15 @@ int resnet_forward(Ctx* c, const ResnetW& w, const ResnetShape& s, NhwcSrc x, co
       return cc.gn && splitk_gn_ok(g2, cc.gn->f);
     };
     const bool fused = gn_fuses(slots, w.c2sk_b);
-    if (w.c2sk_b && !sk_partials_off() && p2.splits > 1 &&
-        (pk.splits > 1 || fused || !gn_fuses(0, w.c2_b))) {
+    bool share = w.c2sk_b && !sk_partials_off() && p2.splits > 1 &&
+                 (pk.splits > 1 || fused || !gn_fuses(0, w.c2_b));
+    if (share) {  // (without memory for the slots the shortcut is a tensor)
+      void* ws = nullptr;
+      rc = workspace(c, slots * rows * s.Cout * sizeof(float), &ws);
+      if (rc && rc != DI_ENOMEM) return rc;
+      share = !rc;
+    }
+    if (share) {
       c2.bias = w.c2sk_b;
       c2.part_slots = slots;
       // the fused GroupNorm reducer reads the partials in column groups

@@ -10,6 +10,8 @@
 
 namespace di {
 
+struct Ctx;
+
 enum AMode { A_DENSE = 0, A_CONV_NHWC = 1, A_CONV_NCHW = 2 };
 enum BMode { B_NK = 0, B_KN = 1 };
 enum Act { ACT_NONE = 0, ACT_GELU = 1, ACT_GEGLU = 2, ACT_SILU = 3, ACT_GELU_TANH = 4 };
@@ -123,6 +125,9 @@ struct GemmArgs {
 // DI_GEMM_SPLITS override, for tuning sweeps).
 GemmPlan gemm_plan(const GemmArgs& g, int elem, int num_cus, int b_mode = B_NK);
 uint64_t gemm_ws_bytes(const GemmArgs& g);
+// Sets g.part to a workspace for the partials of g.splits > 1.  Where there is
+// no memory for them g.splits becomes 1: every problem also runs in one piece.
+int partials_workspace(Ctx* c, GemmArgs& g);
 // Whether the buffer-load (FAST) kernel variant applies.
 bool gemm_fast_ok(const GemmArgs& g, int elem, int a_mode, int b_mode);
 // Byte extent clamped to the buffer-load limit (0 = too large for it).

@@ -122,6 +122,8 @@ int lookup(Ctx* c, di_handle h, Buffer** out);
 
 // Workspace of at least `bytes` (grown with hipMalloc on demand; refused
 // during graph capture, which the owner's warm-up run makes unnecessary).
+// DI_ENOMEM means that there is no memory for it and nothing else: callers that
+// can do without go on with less, every other failure is theirs to pass on.
 int workspace(Ctx* c, uint64_t bytes, void** out);
 // A captured graph takes a reference on the current workspace (returned, may
 // be null) and gives it back when the graph is destroyed.

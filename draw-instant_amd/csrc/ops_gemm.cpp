@@ -6,6 +6,18 @@
 
 using namespace di;
 
+int di::partials_workspace(Ctx* c, GemmArgs& g) {
+  if (g.splits <= 1) return DI_OK;
+  void* ws = nullptr;
+  const int rc = workspace(c, gemm_ws_bytes(g), &ws);
+  if (rc == DI_ENOMEM) {
+    g.splits = 1;
+    return DI_OK;
+  }
+  g.part = (float*)ws;
+  return rc;
+}
+
 namespace {
 
 int run_gemm(di_ctx* ctx, GemmArgs& g, int elem, int a_mode, int b_mode, int tile = -1,
@@ -13,16 +25,8 @@ int run_gemm(di_ctx* ctx, GemmArgs& g, int elem, int a_mode, int b_mode, int til
   const GemmPlan plan = gemm_plan(g, elem, ctx->num_cus, b_mode);
   if (tile < 0) tile = plan.tile;
   g.splits = splits > 0 ? (uint32_t)splits : plan.splits;
-  if (g.splits > 1) {
-    void* ws = nullptr;
-    int rc = workspace(ctx, gemm_ws_bytes(g), &ws);
-    if (rc) {
-      // no memory for the partials: the problem also runs in one piece
-      (void)hipGetLastError();
-      g.splits = 1;
-    }
-    g.part = (float*)ws;
-  }
+  const int rc = partials_workspace(ctx, g);
+  if (rc) return rc;
   launch_gemm(g, elem, a_mode, b_mode, tile, ctx->stream);
   DI_LAUNCH_CHECK();
   return DI_OK;

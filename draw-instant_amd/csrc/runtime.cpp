@@ -105,6 +105,10 @@ int workspace(Ctx* c, uint64_t bytes, void** out) {
              "workspace growth to %llu bytes during graph capture",
              (unsigned long long)bytes);
   uint64_t want = bytes < (1ull << 20) ? (1ull << 20) : bytes;
+  if (const char* lim = getenv("DI_WORKSPACE_LIMIT"))
+    DI_REQUIRE(want <= strtoull(lim, nullptr, 10), DI_ENOMEM,
+               "workspace of %llu bytes would exceed DI_WORKSPACE_LIMIT=%s",
+               (unsigned long long)want, lim);
   DI_HIP(hipStreamSynchronize(c->stream));
   if (c->ws) {
     // A captured graph still writes the old workspace on every replay: keep
@@ -114,7 +118,12 @@ int workspace(Ctx* c, uint64_t bytes, void** out) {
   }
   c->ws = nullptr;
   c->ws_bytes = 0;
-  DI_HIP(hipMalloc(&c->ws, want));
+  if (const hipError_t e = hipMalloc(&c->ws, want); e != hipSuccess) {
+    c->ws = nullptr;
+    if (e == hipErrorOutOfMemory) (void)hipGetLastError();  // handled: not the next launch's
+    DI_REQUIRE(false, e == hipErrorOutOfMemory ? DI_ENOMEM : DI_EHIP,
+               "workspace of %llu bytes: %s", (unsigned long long)want, hipGetErrorString(e));
+  }
   c->ws_bytes = want;
   *out = c->ws;
   return DI_OK;

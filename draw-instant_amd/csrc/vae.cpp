@@ -207,15 +207,8 @@ int gemm16_nk(Ctx* c, const f16* a, uint64_t lda, uint64_t sa, const f16* b, uin
   g.b_bytes = gemm_extent(((uint64_t)(N - 1) * ldb + K) * 2);
   const GemmPlan plan = gemm_plan(g, DI_F16, c->num_cus);
   g.splits = plan.splits;
-  if (g.splits > 1) {
-    void* ws = nullptr;
-    if (workspace(c, gemm_ws_bytes(g), &ws)) {
-      // no memory for the partials: the product also runs in one piece
-      (void)hipGetLastError();
-      g.splits = 1;
-    }
-    g.part = (float*)ws;
-  }
+  const int rc = partials_workspace(c, g);
+  if (rc) return rc;
   launch_gemm(g, DI_F16, A_DENSE, B_NK, plan.tile, c->stream);
   return DI_OK;
 }
