@@ -703,16 +703,17 @@ namespace di {
 // per lane, above that by the workgroup (fp16 4096: 9.2 us for 4096 rows with
 // one wavefront each, 9.8 with four); rows past 8192 fp32 or 16384 fp16
 // values, and rows past 4096 that 16-byte vectors do not fit, take the
-// three-pass kernel.
+// three-pass kernel, as do 2^24 rows or more of one workgroup each (2^32 threads).
 template <typename T>
 static void softmax_dispatch(hipStream_t s, const T* x, T* y, uint32_t inner, uint32_t rows) {
   constexpr int VW = 16 / (int)sizeof(T);
   const unsigned g4 = (rows + 3) / 4;
   const bool vec = (((uintptr_t)x | (uintptr_t)y) & 15) == 0 && inner % VW == 0;
-#define DI_SM(VWV, NVV, WPRV, GRID)                                                  \
-  if (inner <= (uint32_t)(VWV * NVV * WPRV * kWave)) {                               \
-    k_softmax_reg<T, VWV, NVV, WPRV><<<GRID, 256, 0, s>>>(x, y, inner, rows);        \
-    return;                                                                          \
+#define DI_SM(VWV, NVV, WPRV, GRID)                                           \
+  if (inner <= (uint32_t)(VWV * NVV * WPRV * kWave) &&                        \
+      (WPRV == 1 || rows < 1u << 24)) {                                       \
+    k_softmax_reg<T, VWV, NVV, WPRV><<<GRID, 256, 0, s>>>(x, y, inner, rows); \
+    return;                                                                   \
   }
   if (vec) {
     DI_SM(VW, 1, 1, g4)

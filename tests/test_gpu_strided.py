@@ -117,3 +117,28 @@ def test_softmax(dev, rng, inner, dt):
     assert np.isnan(got[4]).all()
     if inner > 2:
         assert np.isnan(got[2, 0]) and np.isnan(got[3]).all()
+
+
+@pytest.fixture
+def large():
+    """A device of its own: buffers of tens of GiB go back with it."""
+    import drawinstant
+    d = drawinstant.Device(0)
+    yield d
+    d.sync()
+    d.destroy()
+
+
+def test_softmax_more_rows_than_workgroups(large):
+    """Rows that a workgroup each would take past 2^32 threads (69 GB)."""
+    rows, inner = (1 << 24) + 3, 2049
+    x = large.create_buffer(rows * inner * 2)
+    large.fill_normal(x, rows * inner, 5, dtype=1)
+    at = [0, 77, rows // 2, (1 << 24) - 1, 1 << 24, rows - 1]
+    src = [large.download(x, np.float16, (inner,), r * inner * 2).astype(np.float64) for r in at]
+    _call(large, "di_softmax", x.handle, x.handle, inner, rows, 1)
+    for r, v in zip(at, src):
+        got = large.download(x, np.float16, (inner,), r * inner * 2).astype(np.float64)
+        e = np.exp(v - v.max())
+        # fp32 arithmetic, one rounding to fp16 (2^-11 relative, 2^-25 below the normals)
+        assert (np.abs(got - e / e.sum()) <= 1.1 * 2.0 ** -11 * e / e.sum() + 2.0 ** -25).all(), r
