@@ -686,9 +686,10 @@ void launch_gather(hipStream_t s, const T* x, T* y, Idx4 c, uint64_t n) {
       }
       z *= c.dim[d];
     }
-    const uint64_t gy = (t.nI + 63) / 64;
-    if (z <= 65535 && gy <= 65535) {
-      k_transpose_tile<T><<<dim3((t.nJ + 63) / 64, (unsigned)gy, (unsigned)z), 256, 0, s>>>(x, y, t);
+    // (the grid: fewer than 2^32 threads along x, 65535 along y and z)
+    const uint64_t gx = ((uint64_t)t.nJ + 63) / 64, gy = ((uint64_t)t.nI + 63) / 64;
+    if (gx < 1u << 24 && gy <= 65535 && z <= 65535) {
+      k_transpose_tile<T><<<dim3((unsigned)gx, (unsigned)gy, (unsigned)z), 256, 0, s>>>(x, y, t);
       return;
     }
   }

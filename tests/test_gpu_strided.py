@@ -142,3 +142,16 @@ def test_softmax_more_rows_than_workgroups(large):
         e = np.exp(v - v.max())
         # fp32 arithmetic, one rounding to fp16 (2^-11 relative, 2^-25 below the normals)
         assert (np.abs(got - e / e.sum()) <= 1.1 * 2.0 ** -11 * e / e.sum() + 2.0 ** -25).all(), r
+
+
+def test_transpose_longer_than_grid(large):
+    """An axis of 2^30 values: its 64 x 64 tiles would take 2^32 threads (34 GB)."""
+    n, r = 1 << 30, 16
+    x, y = large.create_buffer(n * r * 2), large.create_buffer(n * r * 2)
+    large.fill_normal(x, n * r, 6, dtype=1)
+    _call(large, "di_transpose", x.handle, y.handle, 2, _u32([n, r]), _u32([n, 1]), _u32([1, 0]),
+          n * r, 1)
+    w = 5000
+    for c in (0, n // 2 - 7, n - w):
+        ref = np.stack([large.download(x, np.float16, (w,), (i * n + c) * 2) for i in range(r)], 1)
+        assert np.array_equal(large.download(y, np.float16, (w, r), c * r * 2), ref)
