@@ -663,14 +663,16 @@ static GemmPlan f32_plan(const GemmArgs& g, int num_cus) {
     const uint64_t xy = (uint64_t)((g.M + t.bm - 1) / t.bm) * ((g.N + t.bn - 1) / t.bn);
     if (!grid_x_ok(xy, t.id)) continue;
     const uint64_t T = xy * g.batch;
+    const double work = (double)T * stages / num_cus * t.shared;  // least of any split
     for (uint32_t s = 1; s <= 64 && s <= stages && grid_z_ok(g.batch, s); s++) {
       const uint32_t per = (stages + s - 1) / s;
+      const double extra = s > 1 ? 3.0 + (double)g.batch * g.M * g.N * 4.0 * (s + 1) / 3.5e6 : 0.0;
+      if (work + extra > best_t) break;  // and no larger s is less
       if (s > 1 && (per < 2 || (stages + per - 1) / per != s)) continue;
       const uint64_t w = (T * s + num_cus - 1) / num_cus;  // workgroups of the fullest CU
       const uint64_t rem = w % t.res;
-      double us = (double)per * ((double)(w - rem) * t.shared +
-                                 (rem ? std::max(t.alone, rem * t.shared) : 0.0));
-      if (s > 1) us += 3.0 + (double)g.batch * g.M * g.N * 4.0 * (s + 1) / 3.5e6;
+      const double us = (double)per * ((double)(w - rem) * t.shared +
+                                       (rem ? std::max(t.alone, rem * t.shared) : 0.0)) + extra;
       if (us < best_t) {
         best_t = us;
         best = GemmPlan{t.id, s};
@@ -735,13 +737,16 @@ GemmPlan f16_plan(const GemmArgs& g, int num_cus, double* est_us = nullptr) {
         (uint64_t)((g.M + kTileM[t.id] - 1) / kTileM[t.id]) * ((g.N + kTileN[t.id] - 1) / kTileN[t.id]);
     if (!grid_x_ok(xy, t.id)) continue;
     const uint64_t T = xy * g.batch;
+    const double work = t.base + (double)T * stages / num_cus * t.shared;  // least of any split
     for (uint32_t s = 1; s <= 32 && grid_z_ok(g.batch, s); s++) {
       const uint32_t per = (stages + s - 1) / s;
-      if (s > 1 && per < 2) break;
+      const double extra =
+          s > 1 ? 2.5 + 0.1 * s + (double)g.batch * g.M * g.N * 4.0 * (s + 1) / 4.0e6 : 0.0;
+      if ((s > 1 && per < 2) || work + extra > best_t) break;  // and no larger s is less
       if (s > 1 && (stages + per - 1) / per != s) continue;  // an empty split
       const uint64_t w = (T * s + num_cus - 1) / num_cus;  // workgroups of the fullest CU
-      double us = t.base + per * std::max(t.alone, w * t.shared) + (double)(w - 1) * t.epi;
-      if (s > 1) us += 2.5 + 0.1 * s + (double)g.batch * g.M * g.N * 4.0 * (s + 1) / 4.0e6;
+      const double us =
+          t.base + per * std::max(t.alone, w * t.shared) + (double)(w - 1) * t.epi + extra;
       if (us < best_t) {
         best_t = us;
         best = GemmPlan{t.id, s};
@@ -836,6 +841,7 @@ GemmPlan gemm_plan(const GemmArgs& g, int elem, int num_cus, int b_mode) {
   // takes 1.003 of the faster kernel's time on average and 1.13 at most (with
   // equal estimates 1.012 and 1.35).  DI_CONV_BIG=0 turns it off for A/B runs.
   const char* env_big = getenv("DI_CONV_BIG");
+  GemmPlan implicit{-1, 1};  // f16_plan's choice, where it has been asked
   if (elem == DI_F16 && !env_tile && (!env_big || atoi(env_big) != 0) && conv3_big_ok(g) &&
       vec_epi_ok(g, elem, TILE_CONV3_BIG)) {
     const uint32_t tiles = conv3_big_tiles(g);
@@ -846,7 +852,7 @@ GemmPlan gemm_plan(const GemmArgs& g, int elem, int num_cus, int b_mode) {
       other = std::max(1.0, (double)(g.M / 128) * (g.N / 64) * halo.splits / 256.0) * stages /
                   halo.splits * 0.31 + 4.0;
     } else {
-      f16_plan(g, num_cus, &other);
+      implicit = f16_plan(g, num_cus, &other);
     }
     if (tiles >= 85 && big < 1.1 * other) return GemmPlan{TILE_CONV3_BIG, 1};
   }
@@ -861,7 +867,7 @@ GemmPlan gemm_plan(const GemmArgs& g, int elem, int num_cus, int b_mode) {
     return best;
   }
   const bool fast = gemm_fast_ok(g, elem, g.Cin > 0 ? A_CONV_NHWC : A_DENSE, b_mode);
-  best = fast ? f16_plan(g, num_cus) : slow_plan(g, num_cus);
+  best = !fast ? slow_plan(g, num_cus) : implicit.tile >= 0 ? implicit : f16_plan(g, num_cus);
   env_plan_override(g, elem, env_tile, env_split, &best);
   return best;
 }
