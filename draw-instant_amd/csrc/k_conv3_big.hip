@@ -439,7 +439,8 @@ uint32_t conv3_big_tiles(const GemmArgs& g) {
 }
 
 void launch_conv3_big(const GemmArgs& g, hipStream_t s) {
-  // one workgroup per CU of a MI355X, each with a run of tiles
+  // one workgroup per CU of a whole MI355X, each with a run of tiles; a partition
+  // of fewer CUs takes the same runs in turn
   const uint32_t tiles = conv3_big_tiles(g);
   k_conv3_big<<<tiles < 256 ? tiles : 256, 512, 0, s>>>(g);
 }

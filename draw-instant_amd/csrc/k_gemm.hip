@@ -832,7 +832,7 @@ GemmPlan gemm_plan(const GemmArgs& g, int elem, int num_cus, int b_mode) {
   // fastest by these estimates, in microseconds from timings of 22 shapes (us
   // estimated / measured: 512 -> 512 at 96 x 96 61 / 59, at 192 x 192 61 x 3 /
   // 183, 128 -> 128 at 768 x 768 185 / 192, 320 -> 320 at 96 x 96 41 / 39): 0.75
-  // a stage of 256 x 128 x 64 and 7 a tile, in whole rounds of 256 workgroups,
+  // a stage of 256 x 128 x 64 and 7 a tile, in whole rounds of the CUs,
   // against 0.31 a stage of 128 x 64 x 64 for the halo kernel (two per CU: whole
   // rounds do not show) and the implicit GEMM's own plan.  Below that fill the
   // others' smaller tiles win (512 -> 512 at 45 x 66, 60 tiles: 54 against 50
@@ -846,15 +846,15 @@ GemmPlan gemm_plan(const GemmArgs& g, int elem, int num_cus, int b_mode) {
       vec_epi_ok(g, elem, TILE_CONV3_BIG)) {
     const uint32_t tiles = conv3_big_tiles(g);
     const double stages = g.K / 64.0;
-    const double big = ceil(tiles / 256.0) * (stages * 0.75 + 7.0);
+    const double big = ceil((double)tiles / num_cus) * (stages * 0.75 + 7.0);
     double other;
     if (halo.tile >= 0) {
-      other = std::max(1.0, (double)(g.M / 128) * (g.N / 64) * halo.splits / 256.0) * stages /
+      other = std::max(1.0, (double)(g.M / 128) * (g.N / 64) * halo.splits / num_cus) * stages /
                   halo.splits * 0.31 + 4.0;
     } else {
       implicit = f16_plan(g, num_cus, &other);
     }
-    if (tiles >= 85 && big < 1.1 * other) return GemmPlan{TILE_CONV3_BIG, 1};
+    if (tiles >= (uint32_t)num_cus / 3 && big < 1.1 * other) return GemmPlan{TILE_CONV3_BIG, 1};
   }
   if (halo.tile >= 0) return halo;
   if (elem == DI_F16 && tuned_plan(g, &best)) {

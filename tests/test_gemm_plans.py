@@ -88,3 +88,10 @@ def test_large_conv_override_does_not_split(planner):
              for ci, co, h, w in ((576, 64, 30, 31), (64, 128, 16, 16), (1280, 1280, 8, 8))]
     for env in ({}, {"DI_GEMM_SPLITS": "3"}):
         assert planner(probs, DI_GEMM_TILE="15", **env) == [(15, 1)] * len(probs)
+
+
+def test_large_conv_by_the_device_s_cus(planner):
+    """60 tiles are less than a third of 256 CUs, and fill 64."""
+    p = dict(elem=1, M=45 * 66, N=512, K=9 * 512, cin=512, h=45, w=66, ks=3)
+    (whole, _), (part, splits) = planner([p, dict(p, cus=64)])
+    assert whole != 15 and (part, splits) == (15, 1)
