@@ -65,7 +65,7 @@ struct GemmArgs {
   uint32_t splits = 1, k_split = 0;
   uint32_t a_vec_ok = 1, b_vec_ok = 1;  // whole-vector (KV element) loads legal
   // fp32 problem (elem DI_F32) whose B is stored in fp16 and widened exactly
-  // as it loads (fp16-resident weights); bounds-checked kernels only
+  // as it loads (fp16-resident weights)
   int b_f16 = 0;
   // Byte extents of A, A2 (per batch entry) and B for buffer-load range
   // checks; 0 = unknown (generic path).  Must stay below 2 GiB.
@@ -142,8 +142,9 @@ void launch_conv3_halo(const GemmArgs& g, hipStream_t s);
 // The large-image conv kernel (TILE_CONV3_BIG, k_conv3_big.hip): whether it
 // takes this NHWC fp16 conv (3x3, stride 1, pad 1, optional 2x nearest
 // upsample, Cin % 64 == 0, Cout % 64 == 0, any image size, no split-K),
-// whether it can write g.stats (images of a multiple of 64 pixels with at most
-// one 16 x 16 block per 64-pixel slot), its tile count and its launch.
+// whether it can write g.stats (a single image, or images of a multiple of 64
+// pixels, with at most one 16 x 16 block per 64-pixel slot), its tile count and
+// its launch.
 bool conv3_big_ok(const GemmArgs& g);
 bool conv3_big_stats_ok(const GemmArgs& g);
 uint32_t conv3_big_tiles(const GemmArgs& g);

@@ -6,7 +6,8 @@
 // WGSL_FUSED (fused-cross-attn.js:112-173) - without materialising scores:
 // online softmax over 64-key tiles in the exp2 domain.
 //
-// MFMA mapping (v_mfma_f32_16x16x32_f16), one wavefront = 16 queries:
+// MFMA mapping (v_mfma_f32_16x16x32_f16), one wavefront = one or two groups of
+// 16 queries (attn_query_groups):
 //  * S^T = K Q'^T: A = K tile rows (keys) from LDS, B = Q'^T in registers,
 //    where Q' = Q * scale * log2(e) (rounded to fp16 once), so scores come
 //    out in log2 units.  The accumulator starts at -m (the running row max),
@@ -27,10 +28,10 @@
 // the max raised to the tile's and the tile's probabilities recomputed.  Row
 // sums are reduced across the 4 lanes of a query once, at the end.
 //
-// Each workgroup (4 wavefronts = 64 queries) shares double-buffered K / V
-// tiles in LDS (XOR-swizzled 16-byte chunks, conflict-free for the K
-// fragment reads and the transposed V reads; 32 KiB per workgroup, four
-// resident per CU).  The next tile goes straight from memory into LDS
+// Each workgroup (4 wavefronts = 64 queries, 128 with two query groups) shares
+// double-buffered K / V tiles in LDS (XOR-swizzled 16-byte chunks,
+// conflict-free for the K fragment reads and the transposed V reads; 32 KiB
+// per workgroup, four resident per CU, three with two query groups).  The next tile goes straight from memory into LDS
 // (buffer_load ... lds, one 1 KiB row group per instruction, the swizzle
 // applied on the global side) during the MFMAs, by buffer loads whose
 // descriptor ends at the head's last key: keys past Skv (cross-attention's
@@ -123,8 +124,9 @@ __device__ __forceinline__ float sum_q4(float x) {
 // k_attn_combine).
 //
 // QG (1 or 2) groups of 16 queries per wave: with two every K and V fragment
-// read from LDS feeds two MFMAs (64 KiB of reads for 64 x 64 scores are 512
-// clocks of a CU's LDS, their MFMAs 256), for 133 registers instead of 88:
+// read from LDS feeds two MFMAs, half the LDS reads for the same MFMAs (2 x 5
+// heads x 9216: 53.1 M -> 26.5 M LDS clocks, waits on LDS 31.9 M -> 11.8 M wave
+// clocks; the MFMAs are busy 45 % -> 49 % of the clocks), for 133 registers instead of 88:
 // three workgroups of 128 queries per CU instead of four of 64
 // (attn_query_groups).
 //
@@ -540,14 +542,14 @@ uint32_t attn_key_groups(const Ctx* c, uint32_t B, uint32_t H, uint32_t Sq, uint
 
 uint32_t attn_query_groups(const Ctx* c, uint32_t B, uint32_t H, uint32_t Sq, uint32_t Skv,
                            uint32_t splits) {
-  // Two query groups a wave where 64-query workgroups come to more than three a
-  // CU and each walks 20 or more key tiles, 32 or more where the
-  // 128-query ones (three a CU) need a second round.  Measured at the same split
+  // Two query groups a wave where 64-query workgroups come to 3.2 or more a CU
+  // and each walks 20 or more key tiles, 32 or more where the 128-query ones
+  // (three a CU) need a second round.  Measured at the same split
   // count, bit-identical: 1440 workgroups (2 x 5 heads x 9216 queries and keys)
   // 262 -> 222 us, 2560 (8 x 5 x 4096) 199 -> 172, 960 (3 x 5 x 4096) 80.3 ->
   // 72.7, in three ranges (1 x 5 x 4096) 35.3 -> 33.7, 832 (1 x 13 x 4096) 80.0 ->
-  // 72.8.  Half as many workgroups leave CUs short of waves below that (752: 48.9 -> 52.1, 640: 61 -> 67); a
-  // short second round costs more than it gains (1680 of 21 tiles: 49.9 -> 51.8),
+  // 72.8.  Half as many workgroups leave CUs short of waves below that (752:
+  // 48.9 -> 52.1, 640: 61 -> 67); a short second round costs more than it gains (1680 of 21 tiles: 49.9 -> 51.8),
   // and with 16 tiles or the 2 of cross-attention the two are even.
   const uint64_t blocks = (uint64_t)((Sq + 63) / 64) * H * B * splits;
   const uint32_t n = (Skv + BKV - 1) / BKV / splits, cus = (uint32_t)c->num_cus;

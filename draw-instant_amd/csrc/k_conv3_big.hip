@@ -40,12 +40,14 @@
 // bias, activation, residual, store, and the GroupNorm statistics of the stored
 // values.
 //
-// Measured against the implicit GEMM (128 x 128 tiles): 512 -> 512 at 96 x 96
-// 92 -> 59 us, at 192 x 192 257 -> 183 (950 TFLOP/s), 512 -> 512 upsampled to 384 x
-// 384 743 -> 553 (1.26 PFLOP/s), 256 -> 256 at 384 x 384 245 -> 176, 128 -> 128 at
-// 768 x 768 295 -> 195; with residual and SiLU 320 -> 250.  What bounds it: a
-// stage takes 0.75 us for 0.43 us of MFMA at 2.4 GHz, LDS busy for most of it,
-// and a tile's end 7 us that no other workgroup of the CU covers.
+// Measured in turn against the kernels that had these sizes (halo and implicit
+// GEMM): 512 -> 512 at 96 x 96 90 -> 58 us, at 192 x 192 251 -> 182 (955 TFLOP/s),
+// 512 -> 512 upsampled to 384 x 384 781 -> 599 (1.16 PFLOP/s), 256 -> 256 at 384 x
+// 384 250 -> 181, 128 -> 128 at 768 x 768 298 -> 212.  What bounds it: over the
+// clocks of the CUs that hold a tile the MFMAs are busy 67 % (512 channels) and
+// 48 % (128: a tile's end, 7 us that no other workgroup of the CU covers), at the
+// 1.8 GHz that the card runs at here; LDS 38 and 31 %, bank conflicts 11 and 8;
+// waves wait 34 % of theirs, on barriers and the loads behind them.
 #include <type_traits>
 
 #include "di_kernels.h"

@@ -556,10 +556,9 @@ void launch_splitk_reduce_gn(const GemmArgs& g, const GnFuse& f, hipStream_t s) 
 
 const uint32_t kTileM[TILE_COUNT] = {64, 128, 64, 128, 128, 64, 64, 128, 64, 64, 128, 128, 64, 128, 64, 256};
 const uint32_t kTileN[TILE_COUNT] = {64, 64, 128, 128, 160, 160, 64, 64, 128, 128, 64, 128, 64, 64, 32, 128};
-// Relative per-CU MFMA efficiency of each tile shape (the 2x2 wavefront tile
-// sets LDS bytes per MFMA cycle); tuned by measurement.
-const double kTileEff[TILE_COUNT] = {0.35, 0.5, 0.5, 0.8, 0.85, 0.55, 0.35, 0.5, 0.5,
-                                      0.5, 0.5, 0.8, 0.35, 0.8, 0.25, 0.8};
+// Relative per-CU MFMA efficiency of the tiles up to 64 x 128 K2 (slow_plan; the
+// 2x2 wavefront tile sets LDS bytes per MFMA cycle); tuned by measurement.
+const double kTileEff[TILE_64x128_W16] = {0.35, 0.5, 0.5, 0.8, 0.85, 0.55, 0.35, 0.5, 0.5};
 bool vec_epi_ok(const GemmArgs& g, int elem, int tile_cfg);
 
 // What a launch may span: fewer than 2^32 threads along x (a tile's workgroup
@@ -690,13 +689,18 @@ namespace {
 // each of the several that a CU holds (`shared`), the epilogue of each
 // workgroup after a CU's first (`epi`) and the launch with the first one's
 // prologue and epilogue (`base`), for dense operands and for convolutions
-// (whose loads add address work per stage); a split adds its reducer.  Fitted
-// to 9700 timings, every tile and 1-16 splits of 124 dense shapes (64 to 16384
-// rows, K 64 to 5120) and 85 convolutions (1x1 and 3x3, strided and upsampled,
-// 64 to 1920 channels, 8 to 128 pixels a side): its choices take 1.011 of the
-// best plan's time on average and 1.12 at most, where one efficiency per tile
-// and a fixed 1.25 us a workgroup in whole rounds of the chip took 1.17 and
-// 1.52 (5120 x 640 x 2560: 34 -> 26 us; 1280 -> 640 3x3 at 46 x 118: 158 ->
+// (whose loads add address work per stage); a split adds its reducer.  The four
+// are one fit per tile, not four measurements: where a tile's timings do not
+// tell them apart one stands in for another (an `alone` near 0: `base` and
+// `shared` explain all of that tile's timings), so a tile's row is taken over
+// or fitted again as a whole.  Fitted to 9700 timings, every tile and 1-16
+// splits of 124 dense shapes (64 to 16384 rows, K 64 to 5120) and 85
+// convolutions (1x1 and 3x3, strided and upsampled, 64 to 1920 channels, 8 to
+// 128 pixels a side).  What counts is the choice: over the fitted shapes it takes
+// 1.011 of the best plan's time on average and 1.12 at most, over the 38 of
+// profiles/contraction_plan_choices.md 1.02 and 1.13, where one efficiency per
+// tile and a fixed 1.25 us a workgroup in whole rounds of the chip took 1.17
+// and 1.52 (5120 x 640 x 2560: 34 -> 26 us; 1280 -> 640 3x3 at 46 x 118: 158 ->
 // 106; 512 -> 512 3x3 at 2 x 80 x 28: 61 -> 42).  The 64-row tiles of sixteen
 // waves never won and are left to the tuned plans.
 struct TileTime {
@@ -764,9 +768,8 @@ GemmPlan slow_plan(const GemmArgs& g, int num_cus) {
   const double cus = num_cus;
   GemmPlan best{TILE_64x64, 1};
   double best_t = 1e300;
-  for (int tc = 0; tc < TILE_COUNT; tc++) {
+  for (int tc = 0; tc < TILE_64x128_W16; tc++) {
     if (tc == TILE_128x160) continue;  // spills registers: not built
-    if (tc >= TILE_64x128_W16) continue;  // sixteen-wave tiles and conv kernels: chosen above
     if (g.act == ACT_GEGLU && kTileN[tc] == 160) continue;  // GEGLU pairs need even TN
     const uint64_t mt = (g.M + kTileM[tc] - 1) / kTileM[tc], nt = (g.N + kTileN[tc] - 1) / kTileN[tc];
     const uint64_t T = mt * nt * g.batch;

@@ -22,18 +22,20 @@
 //
 // Measured against the fp32 MFMA kernel it replaces (one tile of 128 x 128 or
 // 64 x 64, no split-K, gathered conv loads with divisions per element):
-// conv 3x3 1280 -> 1280 at 16 x 16 967 -> 56 us, linear 2048 x 5120 x 1280
+// conv 3x3 1280 -> 1280 at 16 x 16 969 -> 56 us, linear 2048 x 5120 x 1280
 // 460 -> 165 us and 2048 x 1280 x 5120 470 -> 155 us (170 TFLOP/s of fp32
 // work, a PFLOP/s of bf16; the fp32 MFMA's peak is 157), batched 5 x 2304 x
 // 2304 x 64 90 -> 53 us.  Error against 64 bits (relative 2-norm): 1.4e-6 ->
 // 2.5e-7, 8.0e-7 -> 4.9e-7 over both linears, and between 0.3 and 0.9 times the
-// old kernel's on every shape tried.  The times are those before the scaling,
-// which costs 1 to 3 % (2048 x 5120 x 1280 168.1 -> 171.5 us, 2048 x 1280 x 5120
-// 154.4 -> 157.5, 512 -> 512 at 64 x 64 113.7 -> 117.0 in turn on one card) and
-// without which operands below 2^-110 lost bits: a relative error of 1e-6 at
-// 2^-116, 2e-3 at 2^-126 and 1 at 2^-135, now 1e-7 throughout.  What bounds it is the split-and-store
-// phase (6.5 VALU operations per staged fp32 value) that one workgroup's MFMAs hide
-// from another only in part.
+// old kernel's on every shape tried.  The linears' times are those before the
+// scaling, which costs 1 to 3 % (2048 x 5120 x 1280 168.1 -> 171.5 us, 2048 x
+// 1280 x 5120 154.4 -> 157.5, 512 -> 512 at 64 x 64 113.7 -> 117.0 in turn on one
+// card) and without which operands below 2^-110 lost bits: a relative error of
+// 2e-6 at 2^-116, 2e-3 at 2^-126 and 1 at 2^-135, now 1e-7 throughout.  What
+// bounds it is the split-and-store phase (6.5 VALU operations per staged fp32
+// value, 8.9 VALU instructions with addresses and epilogue) that one workgroup's
+// MFMAs hide from another only in part: the MFMAs are busy 41 to 49 % of the
+// clocks, the LDS 37 to 48 %.
 #include <cstdlib>
 #include <type_traits>
 
@@ -86,8 +88,9 @@ struct F32Tile {
 };
 
 // Byte offset of 16-byte chunk c (8 k) of a row in one part's plane of 64-byte
-// rows: the chunk position is XORed with (row >> 2) & 3, so sixteen rows of
-// one chunk (a fragment read, a k-major store) cover all 64 banks once.
+// rows: the chunk position is XORed with (row >> 2) & 3, which spreads sixteen
+// rows of one chunk (a fragment read, a k-major store) over all 64 banks.  (A
+// third of the LDS's active clocks are bank conflicts all the same.)
 __device__ __forceinline__ uint32_t plane_at(uint32_t row, uint32_t c) {
   return row * 64 + ((c ^ ((row >> 2) & 3)) << 4);
 }
