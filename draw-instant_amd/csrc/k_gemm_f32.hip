@@ -506,7 +506,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f32(GemmArgs g) {
   const bool part = g.splits > 1;
   float* P = part ? g.part + ((uint64_t)split * g.batch + bz) * (uint64_t)g.M * g.N : nullptr;
   const bool geglu = g.act == ACT_GEGLU && !part;
-  // four values of one vector are contiguous and aligned in every tensor
+  // four values of every vector are contiguous and aligned in every tensor
   const bool v4 = A_KMAJ ? g.c_hw % 4 == 0
                          : g.N % 4 == 0 && (part || (g.ldc % 4 == 0 && g.ldr % 4 == 0));
 #pragma unroll
@@ -530,43 +530,71 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f32(GemmArgs g) {
                         gelu_erf_f(epi_value<float>(g, bz, m, n + 16 + j, t[j])));
         continue;
       }
-      if (v4) {
-        uint64_t at, rat;
-        if (A_KMAJ) {  // partials in the output's layout
-          const uint32_t img = m / g.c_hw;
-          rat = at = ((uint64_t)img * g.N + n) * g.c_hw + (m - img * g.c_hw);
-        } else if (part) {
-          rat = at = (uint64_t)m * g.N + n;
-        } else {
-          at = (uint64_t)bz * g.sc + (uint64_t)m * g.ldc + n;
-          rat = (uint64_t)bz * g.sr + (uint64_t)m * g.ldr + n;
+      uint64_t at, rat;
+      uint32_t hw_left = 4;  // pixels of m's image from m on
+      if (A_KMAJ) {  // partials in the output's layout
+        const uint32_t img = m / g.c_hw, p = m - img * g.c_hw;
+        hw_left = g.c_hw - p;
+        rat = at = ((uint64_t)img * g.N + n) * g.c_hw + p;
+      } else if (part) {
+        rat = at = (uint64_t)m * g.N + n;
+      } else {
+        at = (uint64_t)bz * g.sc + (uint64_t)m * g.ldc + n;
+        rat = (uint64_t)bz * g.sr + (uint64_t)m * g.ldr + n;
+      }
+      // The vector's four values go at once, or one by one in straight-line code
+      // where rows or images are no multiple of four (1499 x 10 x 1: 8.3 us with a
+      // loop of one value a turn, 5.5 so, 5.1 the fp32 MFMA kernel; one value a
+      // lane, or 16 bytes wherever a row has them and single values at its end,
+      // took 6.7 and 6.0).
+      uint64_t off[4];
+      bool ok[4];
+      if (!v4) {
+        uint64_t o = 0;
+        uint32_t left = hw_left;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          off[j] = o++;
+          ok[j] = A_KMAJ ? m + j < g.M : n + j < g.N;
+          if (A_KMAJ && --left == 0) {  // the next image's first pixel of this channel
+            o += (uint64_t)(g.N - 1) * g.c_hw;
+            left = g.c_hw;
+          }
         }
-        if (part) {
-          *(f32x4*)(P + at) = v;
-          continue;
-        }
+      }
+      if (!part) {
         f32x4 bias = {0.f, 0.f, 0.f, 0.f};
         if (g.bias) {
-          if (A_KMAJ) bias[0] = bias[1] = bias[2] = bias[3] = g.bias[n];
-          else bias = *(const f32x4*)(g.bias + n);
+          if (A_KMAJ) {
+            bias[0] = bias[1] = bias[2] = bias[3] = g.bias[n];
+          } else if (v4) {
+            bias = *(const f32x4*)(g.bias + n);
+          } else {
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+              if (ok[j]) bias[j] = g.bias[n + j];
+          }
         }
 #pragma unroll
         for (int j = 0; j < 4; j++) v[j] = apply_act(g.act, v[j] * g.alpha + bias[j]);
-        if (g.res) v += *(const f32x4*)((const float*)g.res + rat);
-        *(f32x4*)((float*)g.c + at) = v;
-        continue;
+        if (g.res) {
+          const float* r = (const float*)g.res + rat;
+          if (v4) {
+            v += *(const f32x4*)r;
+          } else {
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+              if (ok[j]) v[j] += r[off[j]];
+          }
+        }
       }
-#pragma unroll 1
-      for (int j = 0; j < 4; j++) {
-        const uint32_t mj = A_KMAJ ? m + j : m, nj = A_KMAJ ? n : n + j;
-        if (mj >= g.M || nj >= g.N) break;
-        const float u = j == 0 ? v[0] : j == 1 ? v[1] : j == 2 ? v[2] : v[3];
-        if (!part)
-          store_out(g, bz, mj, nj, g.N, apply_act(g.act, epi_value<float>(g, bz, mj, nj, u)));
-        else if (A_KMAJ)
-          P[((uint64_t)(mj / g.c_hw) * g.N + nj) * g.c_hw + mj % g.c_hw] = u;
-        else
-          P[(uint64_t)mj * g.N + nj] = u;
+      float* c = part ? P + at : (float*)g.c + at;
+      if (v4) {
+        *(f32x4*)c = v;
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+          if (ok[j]) c[off[j]] = v[j];
       }
     }
   }
