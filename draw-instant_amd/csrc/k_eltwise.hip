@@ -415,8 +415,10 @@ __global__ void k_softmax(const T* __restrict__ x, T* __restrict__ y, uint32_t i
 // VW; elements past the row count as absent), so the row is read and written
 // once, where k_softmax reads it three times.  Memory bound: fp32 11520 rows
 // of 2304 80 -> 31 us (6.9 TB/s, partly from the Infinity Cache), 10240 rows of
-// 77 4.9 -> 4.1 us, fp16 9216 rows of 9216 230 -> 52 us.
-template <typename T, int VW, int NV, int WPR>
+// 77 4.9 -> 4.1 us, fp16 9216 rows of 9216 230 -> 52 us.  FULL: the row has every
+// element, and no load waits for the branch around the one before (fp16 rows of
+// 4096: 243 of them 4.4 -> 3.4 us, 4096 of them 12.5 -> 10.5).
+template <typename T, int VW, int NV, int WPR, bool FULL>
 __global__ __launch_bounds__(256) void k_softmax_reg(const T* __restrict__ x, T* __restrict__ y,
                                                      uint32_t inner, uint32_t rows) {
   typedef T V __attribute__((ext_vector_type(VW)));
@@ -430,8 +432,8 @@ __global__ __launch_bounds__(256) void k_softmax_reg(const T* __restrict__ x, T*
   for (int i = 0; i < NV; i++) {
     const uint32_t at = (i * kWave * WPR + lane) * VW;
     if constexpr (VW == 1) {
-      if (at < inner) v[i][0] = (float)xr[at];
-    } else if (at < inner) {  // inner % VW == 0
+      if (FULL || at < inner) v[i][0] = (float)xr[at];
+    } else if (FULL || at < inner) {  // inner % VW == 0
       const V t = *(const V*)(xr + at);
 #pragma unroll
       for (int e = 0; e < VW; e++) v[i][e] = (float)t[e];
@@ -440,7 +442,7 @@ __global__ __launch_bounds__(256) void k_softmax_reg(const T* __restrict__ x, T*
   float m = -3.0e38f;
 #pragma unroll
   for (int i = 0; i < NV; i++)
-    if ((i * kWave * WPR + lane) * VW < inner)
+    if (FULL || (i * kWave * WPR + lane) * VW < inner)
 #pragma unroll
       for (int e = 0; e < VW; e++) m = fmaxf(m, v[i][e]);
   m = wave_max(m);
@@ -452,7 +454,7 @@ __global__ __launch_bounds__(256) void k_softmax_reg(const T* __restrict__ x, T*
   float s = 0.0f;
 #pragma unroll
   for (int i = 0; i < NV; i++)
-    if ((i * kWave * WPR + lane) * VW < inner)
+    if (FULL || (i * kWave * WPR + lane) * VW < inner)
 #pragma unroll
       for (int e = 0; e < VW; e++) {
         v[i][e] = __expf(v[i][e] - m);
@@ -469,7 +471,7 @@ __global__ __launch_bounds__(256) void k_softmax_reg(const T* __restrict__ x, T*
 #pragma unroll
   for (int i = 0; i < NV; i++) {
     const uint32_t at = (i * kWave * WPR + lane) * VW;
-    if (at < inner) {
+    if (FULL || at < inner) {
       if constexpr (VW == 1) {
         yr[at] = (T)(v[i][0] * inv);
       } else {
@@ -714,11 +716,13 @@ static void softmax_dispatch(hipStream_t s, const T* x, T* y, uint32_t inner, ui
   constexpr int VW = 16 / (int)sizeof(T);
   const unsigned g4 = (rows + 3) / 4;
   const bool vec = (((uintptr_t)x | (uintptr_t)y) & 15) == 0 && inner % VW == 0;
-#define DI_SM(VWV, NVV, WPRV, GRID)                                           \
-  if (inner <= (uint32_t)(VWV * NVV * WPRV * kWave) &&                        \
-      (WPRV == 1 || rows < 1u << 24)) {                                       \
-    k_softmax_reg<T, VWV, NVV, WPRV><<<GRID, 256, 0, s>>>(x, y, inner, rows); \
-    return;                                                                   \
+#define DI_SM(VWV, NVV, WPRV, GRID)                                                        \
+  if (inner <= (uint32_t)(VWV * NVV * WPRV * kWave) && (WPRV == 1 || rows < 1u << 24)) {   \
+    if (inner == (uint32_t)(VWV * NVV * WPRV * kWave))                                     \
+      k_softmax_reg<T, VWV, NVV, WPRV, true><<<GRID, 256, 0, s>>>(x, y, inner, rows);      \
+    else                                                                                   \
+      k_softmax_reg<T, VWV, NVV, WPRV, false><<<GRID, 256, 0, s>>>(x, y, inner, rows);     \
+    return;                                                                                \
   }
   if (vec) {
     DI_SM(VW, 1, 1, g4)
