@@ -531,71 +531,64 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f32(GemmArgs g) {
         continue;
       }
       uint64_t at, rat;
-      uint32_t hw_left = 4;  // pixels of m's image from m on
+      uint32_t left = 4;  // pixels of m's image from m on
       if (A_KMAJ) {  // partials in the output's layout
-        const uint32_t img = m / g.c_hw, p = m - img * g.c_hw;
-        hw_left = g.c_hw - p;
-        rat = at = ((uint64_t)img * g.N + n) * g.c_hw + p;
+        const uint32_t img = m / g.c_hw;
+        rat = at = ((uint64_t)img * g.N + n) * g.c_hw + (m - img * g.c_hw);
+        left = g.c_hw - (m - img * g.c_hw);
       } else if (part) {
         rat = at = (uint64_t)m * g.N + n;
       } else {
         at = (uint64_t)bz * g.sc + (uint64_t)m * g.ldc + n;
         rat = (uint64_t)bz * g.sr + (uint64_t)m * g.ldr + n;
       }
-      // The vector's four values go at once, or one by one in straight-line code
-      // where rows or images are no multiple of four (1499 x 10 x 1: 8.3 us with a
-      // loop of one value a turn, 5.5 so, 5.1 the fp32 MFMA kernel; one value a
-      // lane, or 16 bytes wherever a row has them and single values at its end,
-      // took 6.7 and 6.0).
-      uint64_t off[4];
-      bool ok[4];
-      if (!v4) {
-        uint64_t o = 0;
-        uint32_t left = hw_left;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          off[j] = o++;
-          ok[j] = A_KMAJ ? m + j < g.M : n + j < g.N;
-          if (A_KMAJ && --left == 0) {  // the next image's first pixel of this channel
-            o += (uint64_t)(g.N - 1) * g.c_hw;
-            left = g.c_hw;
-          }
+      if (v4) {
+        if (part) {
+          *(f32x4*)(P + at) = v;
+          continue;
         }
-      }
-      if (!part) {
         f32x4 bias = {0.f, 0.f, 0.f, 0.f};
         if (g.bias) {
-          if (A_KMAJ) {
-            bias[0] = bias[1] = bias[2] = bias[3] = g.bias[n];
-          } else if (v4) {
-            bias = *(const f32x4*)(g.bias + n);
-          } else {
-#pragma unroll
-            for (int j = 0; j < 4; j++)
-              if (ok[j]) bias[j] = g.bias[n + j];
-          }
+          if (A_KMAJ) bias[0] = bias[1] = bias[2] = bias[3] = g.bias[n];
+          else bias = *(const f32x4*)(g.bias + n);
         }
 #pragma unroll
         for (int j = 0; j < 4; j++) v[j] = apply_act(g.act, v[j] * g.alpha + bias[j]);
-        if (g.res) {
-          const float* r = (const float*)g.res + rat;
-          if (v4) {
-            v += *(const f32x4*)r;
-          } else {
+        if (g.res) v += *(const f32x4*)((const float*)g.res + rat);
+        *(f32x4*)((float*)g.c + at) = v;
+        continue;
+      }
+      // Rows or images of no multiple of four: one by one, in straight-line code
+      // (137 x 562 x 18 8.6 us with a loop of one value a turn, 6.1 so; one value
+      // a lane, or 16 bytes wherever a row has them and single values at its end,
+      // took 7.0 and 6.1, but 6.7 and 6.0 against 5.6 for 1499 x 10 x 1).
+      uint64_t off[4], o = 0;
+      bool ok[4];
 #pragma unroll
-            for (int j = 0; j < 4; j++)
-              if (ok[j]) v[j] += r[off[j]];
-          }
+      for (int j = 0; j < 4; j++) {
+        off[j] = o++;
+        ok[j] = A_KMAJ ? m + j < g.M : n + j < g.N;
+        if (A_KMAJ && --left == 0) {  // the next image's first pixel of this channel
+          o += (uint64_t)(g.N - 1) * g.c_hw;
+          left = g.c_hw;
         }
       }
-      float* c = part ? P + at : (float*)g.c + at;
-      if (v4) {
-        *(f32x4*)c = v;
-      } else {
+      if (!part) {
 #pragma unroll
-        for (int j = 0; j < 4; j++)
-          if (ok[j]) c[off[j]] = v[j];
+        for (int j = 0; j < 4; j++) {
+          const float bias = g.bias && ok[j] ? g.bias[A_KMAJ ? n : n + j] : 0.0f;
+          v[j] = apply_act(g.act, v[j] * g.alpha + bias);
+        }
+        if (g.res) {
+#pragma unroll
+          for (int j = 0; j < 4; j++)
+            if (ok[j]) v[j] += ((const float*)g.res + rat)[off[j]];
+        }
       }
+      float* c = (part ? P : (float*)g.c) + at;
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+        if (ok[j]) c[off[j]] = v[j];
     }
   }
 }
@@ -677,6 +670,13 @@ bool gemm_f32_ok(const GemmArgs& g, int a_mode, int b_mode) {
   // its first row (its first image; its stage's first k)
   const uint64_t lim = 0x7fff0000ull;
   if (!g.c_f32 || (g.res && !g.res_f32) || g.bias2) return false;
+  // Narrow shallow products whose rows are no multiple of four stay with the
+  // fp32 MFMA, which stores such rows straight from its accumulators: up to 15
+  // columns and K of 31 (B k-major) or 64, M of 64 to 8192, its time is 0.88 to
+  // 0.98 of this kernel's; even at K = 32 and 96 and from there on, and from 17
+  // columns on, this one is the faster (1.1 to 3.5).
+  if (a_mode == A_DENSE && g.N < 16 && g.N % 4 != 0 && g.K <= (b_mode == B_KN ? 31u : 64u))
+    return false;
   if (a_mode == A_CONV_NCHW) {
     const uint64_t hw = (uint64_t)g.Ho * g.Wo, img = (uint64_t)g.Cin * g.H * g.W * 4;
     if ((127 / hw + 2) * img > lim || (g.up != 1 && g.up != 2)) return false;

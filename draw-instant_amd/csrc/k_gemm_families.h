@@ -21,8 +21,8 @@ void gemm_fast_conv(const GemmArgs& g, int tile_cfg, hipStream_t s);
 bool gemm_f32_ok(const GemmArgs& g, int a_mode, int b_mode);
 void gemm_f32(const GemmArgs& g, int a_mode, int b_mode, int tile_cfg, hipStream_t s);
 // Bounds-checked kernels: fp16 (dense / B_KN / NHWC conv), fp32 and fp32
-// with fp16-resident B (dense / B_KN / NCHW conv) past gemm_f32_ok's
-// operand sizes (k_gemm_slow.hip).
+// with fp16-resident B (dense / B_KN / NCHW conv) that gemm_f32_ok does not
+// take: operands past its offsets, narrow shallow products (k_gemm_slow.hip).
 void gemm_slow(const GemmArgs& g, int elem, int a_mode, int b_mode, int tile_cfg, hipStream_t s);
 
 }  // namespace di

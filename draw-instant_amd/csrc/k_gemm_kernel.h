@@ -13,7 +13,7 @@
 //  * the reference's fp32 ops (matmul wgsl-ops.js:477-556, gemm :821-897,
 //    convMM :584-698 with its (ci, ky, kx) k order on NCHW) through an fp32
 //    MFMA variant with exact fp32 products, where an operand is too large for
-//    k_gemm_f32.hip.
+//    k_gemm_f32.hip or the product too small to gain from it.
 // Epilogue: alpha, per-column bias, per-(batch, column) bias (ResNet temb),
 // residual add, GELU(erf) / GEGLU / SiLU, fp16 or fp32 store, NHWC or NCHW.
 //
@@ -1216,8 +1216,7 @@ void launch_cfg(const GemmArgs& g, hipStream_t s) {
       <<<dim3(tiles, 1, g.batch * g.splits), 64 * WGM * WGN * KS, 0, s>>>(g);
 }
 
-// Generic (bounds-checked) variants: two tile shapes.  fp32 (operands past the
-// split kernel's 31-bit offsets) takes the larger one only where 64 x 64 tiles
+// Generic (bounds-checked) variants: two tile shapes.  fp32 takes the larger one only where 64 x 64 tiles
 // would pass the grid's 2^32 threads (128 -> 3 channels at 1536 x 1536: 6.8 ms on
 // 64 x 64, 16.1 on 128 x 128; 128 -> 128 13.8 and 17.3).
 template <typename T, int AM, int BMD, typename TB = T>

@@ -1,6 +1,6 @@
 // k_gemm instantiations: the bounds-checked kernels (fp16 operands the
-// buffer-load path does not take; fp32 ops, with fp32 or fp16-resident B, on
-// operands too large for k_gemm_f32.hip).
+// buffer-load path does not take; fp32 ops, with fp32 or fp16-resident B, that
+// k_gemm_f32.hip does not).
 #include "k_gemm_families.h"
 #include "k_gemm_kernel.h"
 

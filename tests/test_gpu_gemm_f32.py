@@ -238,3 +238,38 @@ def test_tile_override(dev, rng, monkeypatch, tile):
         _call(dev, "di_gemm", dev.storage(a).handle, dev.storage(b).handle, 0, y.handle, M, N, K, 1, F32)
         a64, b64 = a.astype(np.float64), b.astype(np.float64)
         _check(dev.download(y).reshape(M, N), a64 @ b64.T, np.abs(a64) @ np.abs(b64).T, K)
+
+
+@pytest.mark.parametrize("trans_b", [0, 1])
+@pytest.mark.parametrize("M,N,K", [(240, 5, 2), (65, 15, 31), (65, 15, 32), (130, 13, 64), (130, 13, 65),
+                                   (64, 16, 20), (3, 1, 8)])
+def test_narrow(dev, rng, M, N, K, trans_b):
+    """Both sides of the line up to which the fp32 MFMA takes narrow products."""
+    a, b = _mats(rng, (M, K), (N, K) if trans_b else (K, N))
+    c = rng.standard_normal(N).astype(np.float32)
+    y = dev.create_buffer(M * N * 4)
+    _call(dev, "di_gemm", dev.storage(a).handle, dev.storage(b).handle, dev.storage(c).handle,
+          y.handle, M, N, K, trans_b, F32)
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    b64 = b64.T if trans_b else b64
+    _check(dev.download(y).reshape(M, N), a64 @ b64 + c, np.abs(a64) @ np.abs(b64) + np.abs(c), K)
+
+
+@pytest.mark.parametrize("N,co,H,W,silu", [(3, 66, 1, 1, 0), (2, 70, 1, 3, SILU), (5, 5, 3, 3, 0),
+                                           (2, 130, 5, 5, SILU)])
+def test_ragged_images(dev, rng, N, co, H, W, silu):
+    """Images of no multiple of four pixels: a stored vector spans one to four."""
+    ci = 40
+    x = rng.standard_normal((N, ci, H, W)).astype(np.float32)
+    w = rng.standard_normal((co, ci, 3, 3)).astype(np.float32)
+    b = rng.standard_normal(co).astype(np.float32)
+    r = rng.standard_normal((N, co, H, W)).astype(np.float32)
+    y = dev.create_buffer(r.size * 4)
+    _call(dev, "di_conv2d", dev.storage(x).handle, dev.storage(w).handle, dev.storage(b).handle,
+          dev.storage(r).handle, y.handle, N, ci, co, H, W, 3, 1, 1, silu, F32, NCHW)
+    t = [torch.from_numpy(v.astype(np.float64)) for v in (x, w, b)]
+    z = TF.conv2d(*t, padding=1).numpy()
+    mag = TF.conv2d(*(v.abs() for v in t), padding=1).numpy()
+    ref = (z / (1 + np.exp(-z)) if silu else z) + r
+    _check(dev.download(y).reshape(r.shape), ref, 1.1 * mag + np.abs(r), ci * 9,
+           2.0 ** -20 * np.abs(z) if silu else 0.0)
