@@ -33,10 +33,11 @@ void gn_exchange_area(Ctx* c, GnFuse& f) {
 
 int run(Ctx* c, GemmArgs& g, int a_mode, StatsOut* st = nullptr, RowStatsOut* rst = nullptr,
         GnFuseOut* gn = nullptr) {
+  g.stats = nullptr;
+  g.rstats = rst ? rst->p : nullptr;  // the plan prefers tiles that write them
   const GemmPlan plan = gemm_plan(g, DI_F16, c->num_cus);
   const int tile = plan.tile;
   g.splits = plan.splits;
-  g.stats = nullptr;
   g.rstats = nullptr;
   // before anything that depends on whether the problem splits; slots shared
   // with another launch were reserved by the caller

@@ -689,20 +689,24 @@ namespace {
 // each of the several that a CU holds (`shared`), the epilogue of each
 // workgroup after a CU's first (`epi`) and the launch with the first one's
 // prologue and epilogue (`base`), for dense operands and for convolutions
-// (whose loads add address work per stage); a split adds its reducer.  The four
-// are one fit per tile, not four measurements: where a tile's timings do not
-// tell them apart one stands in for another (an `alone` near 0: `base` and
-// `shared` explain all of that tile's timings), so a tile's row is taken over
-// or fitted again as a whole.  Fitted to 9700 timings, every tile and 1-16
-// splits of 124 dense shapes (64 to 16384 rows, K 64 to 5120) and 85
-// convolutions (1x1 and 3x3, strided and upsampled, 64 to 1920 channels, 8 to
-// 128 pixels a side).  What counts is the choice: over the fitted shapes it takes
-// 1.011 of the best plan's time on average and 1.12 at most, over the 38 of
-// profiles/contraction_plan_choices.md 1.02 and 1.13, where one efficiency per
-// tile and a fixed 1.25 us a workgroup in whole rounds of the chip took 1.17
-// and 1.52 (5120 x 640 x 2560: 34 -> 26 us; 1280 -> 640 3x3 at 46 x 118: 158 ->
-// 106; 512 -> 512 3x3 at 2 x 80 x 28: 61 -> 42).  The 64-row tiles of sixteen
-// waves never won and are left to the tuned plans.
+// (whose loads add address work per stage, 1x1 ones too); a split adds its
+// reducer.  The four are one fit per tile, not four measurements: where a tile's
+// timings do not tell them apart one stands in for another (an `alone` near 0:
+// `base` and `shared` explain all of that tile's timings), so a tile's row is
+// taken over or fitted again as a whole.  The rows were first fitted to 9700
+// timings of single plans and then moved, in a random search, to the least sum
+// of chosen / best plan over 3370 drawn shapes timed with every tile and 1-16
+// splits (32 to 16384 rows, K 64 to 8192, the U-Net's own projections among them;
+// 1x1 and 3x3 convolutions, strided and upsampled, 64 to 1920 channels, 8 to 128
+// pixels a side).  What counts is the choice: over 1680 other shapes it takes
+// 1.007 of the best plan's time on average and 1.05 or more in 1 of 20
+// (profiles/contraction_plan_choices.md); one efficiency per tile and a fixed
+// 1.25 us a workgroup in whole rounds of the chip took 1.2 times this planner's
+// (5120 x 640 x 2560: 34 -> 26 us; 1280 -> 640 3x3 at 46 x 118: 158 -> 106; 512 ->
+// 512 3x3 at 2 x 80 x 28: 61 -> 42).  (A first table without the 64 x 160 tile and
+// with 1x1 convolutions timed as dense lost up to 19 % to that: 3270 x 1280 x 2560
+// 38 and 47 us, 1920 -> 320 1x1 at 17 x 17 9.5 and 11.1.)  The 64-row tiles of
+// sixteen waves never won and are left to the tuned plans.
 struct TileTime {
   int id;
   double alone, shared, epi, base;
@@ -710,31 +714,36 @@ struct TileTime {
 
 GemmPlan f16_plan(const GemmArgs& g, int num_cus, double* est_us = nullptr) {
   static const TileTime dense[] = {{TILE_64x64, 0.23, 0.197, 0.45, 4.3},
-                                   {TILE_128x64, 0.40, 0.336, 0.9, 5.2},
-                                   {TILE_64x128, 0.38, 0.317, 0.95, 5.1},
-                                   {TILE_128x128, 0.38, 0.585, 1.55, 6.6},
+                                   {TILE_128x64, 0.40, 0.305, 0.97, 6.4},
+                                   {TILE_64x128, 0.38, 0.317, 0.65, 5.7},
+                                   {TILE_128x128, 0.38, 0.517, 2.08, 7.45},
                                    {TILE_64x64_K2, 0.15, 0.175, 0.85, 4.35},
-                                   {TILE_128x64_K2, 0.31, 0.303, 1.35, 4.85},
-                                   {TILE_64x128_K2, 0.02, 0.302, 1.3, 5.0},
-                                   {TILE_128x64_W16, 0.29, 0.31, 3.0, 4.85},
-                                   {TILE_128x128_W16, 0.06, 0.473, 5.5, 6.1},
-                                   {TILE_64x32_K2, 0.11, 0.123, 0.5, 4.35}};
+                                   {TILE_128x64_K2, 0.31, 0.294, 1.60, 4.4},
+                                   {TILE_64x128_K2, 0.02, 0.276, 1.55, 5.25},
+                                   {TILE_128x64_W16, 0.29, 0.279, 5.0, 4.5},
+                                   {TILE_128x128_W16, 0.06, 0.487, 7.3, 6.65},
+                                   {TILE_64x32_K2, 0.11, 0.123, 0.5, 4.35},
+                                   {TILE_64x160, 0.45, 0.347, 1.85, 7.7}};
   static const TileTime conv[] = {{TILE_64x64, 0.30, 0.198, 0.15, 5.45},
-                                  {TILE_128x64, 0.51, 0.341, 0.9, 6.1},
-                                  {TILE_64x128, 0.45, 0.323, 0.25, 6.0},
-                                  {TILE_128x128, 0.70, 0.484, 1.1, 7.1},
+                                  {TILE_128x64, 0.51, 0.354, 0.54, 6.25},
+                                  {TILE_64x128, 0.45, 0.324, 0.24, 5.6},
+                                  {TILE_128x128, 0.70, 0.512, 1.76, 5.95},
                                   {TILE_64x64_K2, 0.23, 0.188, 0.75, 5.1},
-                                  {TILE_128x64_K2, 0.39, 0.298, 1.0, 5.7},
-                                  {TILE_64x128_K2, 0.33, 0.292, 0.8, 5.7},
-                                  {TILE_128x64_W16, 0.01, 0.36, 2.7, 5.95},
-                                  {TILE_128x128_W16, 0.03, 0.496, 4.0, 7.0},
-                                  {TILE_64x32_K2, 0.22, 0.144, 0.5, 5.05}};
-  const bool is_conv = g.Cin > 0 && g.ks > 1;
+                                  {TILE_128x64_K2, 0.39, 0.305, 0.77, 5.6},
+                                  {TILE_64x128_K2, 0.33, 0.297, 1.02, 5.55},
+                                  {TILE_128x64_W16, 0.01, 0.355, 4.16, 5.85},
+                                  {TILE_128x128_W16, 0.03, 0.502, 4.17, 6.25},
+                                  {TILE_64x32_K2, 0.22, 0.144, 0.5, 5.05},
+                                  {TILE_64x160, 0.60, 0.407, 0.69, 6.6}};
+  const bool is_conv = g.Cin > 0;
   const uint32_t stages = g.K / 64;
   GemmPlan best{TILE_128x128, 1};
   double best_t = 1e300;
-  for (int i = 0; i < 10; i++) {
+  for (int i = 0; i < 11; i++) {
     const TileTime& t = is_conv ? conv[i] : dense[i];
+    // no row statistics from 160 columns, five fragments to a wave that GEGLU
+    // cannot pair
+    if (t.id == TILE_64x160 && (g.rstats || g.act == ACT_GEGLU)) continue;
     // 16 columns to a wave: only the vector epilogue pairs GEGLU's columns
     if (t.id == TILE_64x32_K2 && g.act == ACT_GEGLU && !vec_epi_ok(g, DI_F16, t.id)) continue;
     const uint64_t xy =

@@ -7,11 +7,13 @@
 
 int main() {
   // elem (0 fp32, 1 fp16), b_mode, CUs, batch, M, N, K, act, then for a conv its
-  // input channels (0: dense), size, kernel, stride and upsampling
-  unsigned elem, b_mode, cus, batch, M, N, K, act, cin, h, w, ks, stride, up;
-  while (scanf("%u %u %u %u %u %u %u %u %u %u %u %u %u %u", &elem, &b_mode, &cus, &batch, &M, &N,
-               &K, &act, &cin, &h, &w, &ks, &stride, &up) == 14) {
+  // input channels (0: dense), size, kernel, stride and upsampling, and whether
+  // row statistics are wanted
+  unsigned elem, b_mode, cus, batch, M, N, K, act, cin, h, w, ks, stride, up, rstats;
+  while (scanf("%u %u %u %u %u %u %u %u %u %u %u %u %u %u %u", &elem, &b_mode, &cus, &batch, &M, &N,
+               &K, &act, &cin, &h, &w, &ks, &stride, &up, &rstats) == 15) {
     di::GemmArgs g;
+    if (rstats) g.rstats = (float*)4096;
     const uint64_t es = elem ? 2 : 4;
     g.a = g.b = g.c = (void*)4096;
     g.batch = batch;

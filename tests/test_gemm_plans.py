@@ -33,11 +33,12 @@ def planner(tmp_path_factory):
         """(tile, splits) of each problem: dicts of gemm_plan_check's fields."""
         rows = []
         for p in problems:
-            q = dict(elem=0, b_mode=0, cus=256, batch=1, act=0, cin=0, h=0, w=0, ks=1, stride=1, up=1)
+            q = dict(elem=0, b_mode=0, cus=256, batch=1, act=0, cin=0, h=0, w=0, ks=1, stride=1, up=1,
+                     rstats=0)
             q.update(p)
             rows.append(" ".join(str(int(q[k])) for k in (
                 "elem", "b_mode", "cus", "batch", "M", "N", "K", "act", "cin", "h", "w", "ks",
-                "stride", "up")))
+                "stride", "up", "rstats")))
         r = subprocess.run([str(exe)], input="\n".join(rows) + "\n", capture_output=True, text=True,
                            timeout=120, env={**os.environ, **env}, check=True)
         out = [tuple(int(v) for v in ln.split()) for ln in r.stdout.splitlines()]
@@ -95,3 +96,21 @@ def test_large_conv_by_the_device_s_cus(planner):
     p = dict(elem=1, M=45 * 66, N=512, K=9 * 512, cin=512, h=45, w=66, ks=3)
     (whole, _), (part, splits) = planner([p, dict(p, cus=64)])
     assert whole != 15 and (part, splits) == (15, 1)
+
+
+def test_columns_of_160(planner):
+    """Sizes where the 64 x 160 tile is the fastest by 4 to 15 % (N of whole 160s,
+    deep K, more than a round of the chip), unless its rows' statistics are wanted,
+    which it cannot write; and none of it for GEGLU."""
+    probs = [dict(elem=1, M=m, N=n, K=k) for m, n, k in ((3270, 1280, 2560), (3713, 1280, 2560),
+                                                         (8016, 640, 2560), (14456, 320, 2560))]
+    assert [t for t, _ in planner(probs)] == [5] * 4
+    assert 5 not in [t for t, _ in planner([dict(p, rstats=1) for p in probs])]
+    assert 5 not in [t for t, _ in planner([dict(p, act=2) for p in probs])]
+
+
+def test_deep_1x1_convolutions_split(planner):
+    """1x1 convolutions of small images over many channels: a split saves 10 to 25 %."""
+    probs = [dict(elem=1, M=h * w, N=co, K=1920, cin=1920, h=h, w=w)
+             for co, h, w in ((320, 17, 17), (640, 26, 7), (152, 12, 29))]
+    assert all(s > 1 for _, s in planner(probs))
