@@ -12,10 +12,12 @@
 namespace di {
 
 struct AttnArgs {
-  const f16* q = nullptr;
-  const f16* k = nullptr;
-  const f16* v = nullptr;
-  f16* o = nullptr;
+  // fp16, or fp32 as `f32` says (one set of pointers: the kernels read their
+  // arguments first)
+  const void* q = nullptr;
+  const void* k = nullptr;
+  const void* v = nullptr;
+  void* o = nullptr;
   uint64_t ldq = 0, ldk = 0, ldv = 0, ldo = 0;  // token row stride
   uint64_t hq = 0, hk = 0, hv = 0, ho = 0;      // head stride
   uint64_t bq = 0, bk = 0, bv = 0, bo = 0;      // batch stride
@@ -30,12 +32,8 @@ struct AttnArgs {
   uint32_t key_groups = 1;
   // 16-query groups per wave (1 or 2; set by run_attention)
   uint32_t query_groups = 1;
-  // fp32 tensors: q32 / o32 (strides as q / o, in elements) take the place of
-  // q / o, and k32 / v32 of k / v; null: the fp16 pointers
-  const float* q32 = nullptr;
-  const float* k32 = nullptr;
-  const float* v32 = nullptr;
-  float* o32 = nullptr;
+  // fp32 tensors: 0 none, 1 queries and outputs, 2 keys and values too
+  uint32_t f32 = 0;
   uint64_t rows = 0;
   f16* part_o = nullptr;
   float* part_ml = nullptr;

@@ -152,11 +152,12 @@ __global__ __launch_bounds__(256 * KS, QG == 1 ? 4 : 3) void k_flash_attn(AttnAr
   const uint32_t qb = w % nqb, rest = w / nqb, split = rest % a.splits, hb = rest / a.splits;
   const uint32_t h = hb % a.H, b = hb / a.H;
 
+  typedef typename std::conditional<IO == 0, f16, float>::type QT;
   typedef typename std::conditional<IO == 2, float, f16>::type KT;
-  const uint64_t qo = b * a.bq + h * a.hq;
-  const KT* K = (IO == 2 ? (const KT*)a.k32 : (const KT*)a.k) + b * a.bk + h * a.hk;
-  const KT* V = (IO == 2 ? (const KT*)a.v32 : (const KT*)a.v) + b * a.bv + h * a.hv;
-  const uint64_t oo = b * a.bo + h * a.ho;
+  const QT* Q = (const QT*)a.q + b * a.bq + h * a.hq;
+  const KT* K = (const KT*)a.k + b * a.bk + h * a.hk;
+  const KT* V = (const KT*)a.v + b * a.bv + h * a.hv;
+  QT* O = (QT*)a.o + b * a.bo + h * a.ho;
 
   // Q'^T fragments for the two 32-wide d steps
   const uint32_t qrow0 = qb * (64 * QG) + wave * (16 * QG) + r;
@@ -167,11 +168,11 @@ __global__ __launch_bounds__(256 * KS, QG == 1 ? 4 : 3) void k_flash_attn(AttnAr
     const uint32_t qrow = qrow0 + qi * 16;
     f16x8 t = {};
     if (qrow < a.Sq) {
-      const uint64_t at = qo + (uint64_t)qrow * a.ldq + ks * 32 + g * 8;
+      const QT* p = Q + (uint64_t)qrow * a.ldq + ks * 32 + g * 8;
       if constexpr (IO == 0) {
-        t = *(const f16x8*)(a.q + at);
+        t = *(const f16x8*)p;
       } else {
-        const f32x4 lo = *(const f32x4*)(a.q32 + at), hi = *(const f32x4*)(a.q32 + at + 4);
+        const f32x4 lo = *(const f32x4*)p, hi = *(const f32x4*)(p + 4);
 #pragma unroll
         for (int j = 0; j < 4; j++) {
           t[j] = (f16)lo[j];
@@ -431,13 +432,15 @@ __global__ __launch_bounds__(256 * KS, QG == 1 ? 4 : 3) void k_flash_attn(AttnAr
     const uint32_t qrow = qrow0 + qi * 16;
     if (qrow >= a.Sq) break;
     const float inv = 1.0f / l[qi];
-    if (IO > 0 && a.splits == 1) {
-      float* d32 = a.o32 + oo + (uint64_t)qrow * a.ldo;
+    if constexpr (IO > 0) {
+      if (a.splits == 1) {
+        float* d32 = O + (uint64_t)qrow * a.ldo;
 #pragma unroll
-      for (int dt = 0; dt < 4; dt++) *(f32x4*)(d32 + dt * 16 + g * 4) = o[qi][dt] * inv;
-      continue;
+        for (int dt = 0; dt < 4; dt++) *(f32x4*)(d32 + dt * 16 + g * 4) = o[qi][dt] * inv;
+        continue;
+      }
     }
-    f16* dst = IO > 0 ? nullptr : a.o + oo + (uint64_t)qrow * a.ldo;
+    f16* dst = IO > 0 ? nullptr : (f16*)O + (uint64_t)qrow * a.ldo;
     if (a.splits > 1) {
       // this key range's normalised output and (max, row sum), per row
       // (b, h, q) of the [splits][B*H*Sq] workspace
@@ -487,13 +490,13 @@ __global__ __launch_bounds__(256) void k_attn_combine(AttnArgs a) {
   if constexpr (F32) {
 #pragma unroll
     for (int j = 0; j < 8; j += 4)
-      *(f32x4*)(a.o32 + at + j) =
+      *(f32x4*)((float*)a.o + at + j) =
           f32x4{acc[j] * inv, acc[j + 1] * inv, acc[j + 2] * inv, acc[j + 3] * inv};
   } else {
     f16x8 out;
 #pragma unroll
     for (int j = 0; j < 8; j++) out[j] = (f16)(acc[j] * inv);
-    *(f16x8*)(a.o + at) = out;
+    *(f16x8*)((f16*)a.o + at) = out;
   }
 }
 
@@ -595,10 +598,10 @@ static void launch_combine(const AttnArgs& a, hipStream_t s) {
 }
 
 void launch_attention(const AttnArgs& a, uint32_t B, hipStream_t s) {
-  if (!a.q32) launch_flash<0>(a, B, s);
-  else if (!a.k32) launch_flash<1>(a, B, s);
+  if (a.f32 == 0) launch_flash<0>(a, B, s);
+  else if (a.f32 == 1) launch_flash<1>(a, B, s);
   else launch_flash<2>(a, B, s);
-  if (a.q32) launch_combine<true>(a, s);
+  if (a.f32) launch_combine<true>(a, s);
   else launch_combine<false>(a, s);
 }
 
@@ -686,11 +689,11 @@ int attention_entry(di_ctx* ctx, di_handle Q, di_handle K, di_handle V, di_handl
   a.ldo = a.ldq;
   a.ho = a.hq;
   a.bo = a.bq;
+  a.q = q->ptr;
+  a.k = k->ptr;
+  a.v = v->ptr;
+  a.o = o->ptr;
   if (dt == DI_F16) {
-    a.q = (const f16*)q->ptr;
-    a.k = (const f16*)k->ptr;
-    a.v = (const f16*)v->ptr;
-    a.o = (f16*)o->ptr;
     const int rc = run_attention(ctx, a, B);
     if (rc) return rc;
     DI_LAUNCH_CHECK();
@@ -704,13 +707,10 @@ int attention_entry(di_ctx* ctx, di_handle Q, di_handle K, di_handle V, di_handl
   // one out around the fp16 kernel: B2 H20 256 x 77 16.4 -> 5.3 us, 512 x 512
   // (H20) 18.4 -> 8.7, 1024 x 1024 (B2 H10) 28.7 -> 19.9, B2 H5 9216 x 9216
   // 297 -> 281.
-  a.q32 = (const float*)q->ptr;
-  a.o32 = (float*)o->ptr;
   // (An output over the keys' or values' own buffer needs them read first.)
   if (Skv <= 8 * BKV && o->ptr != k->ptr && o->ptr != v->ptr &&
       (uint64_t)(Skv + BKV) * a.ldk * 4 < (1ull << 31)) {
-    a.k32 = (const float*)k->ptr;
-    a.v32 = (const float*)v->ptr;
+    a.f32 = 2;
     const int rc = run_attention(ctx, a, B);
     if (rc) return rc;
     DI_LAUNCH_CHECK();
@@ -720,8 +720,9 @@ int attention_entry(di_ctx* ctx, di_handle Q, di_handle K, di_handle V, di_handl
   uint64_t cap = 0;
   int rc = pool_alloc(ctx, nkv * 4, &tkv, &cap);
   if (rc) return rc;
-  a.k = (const f16*)tkv;
-  a.v = a.k + nkv;
+  a.f32 = 1;
+  a.k = tkv;
+  a.v = (const f16*)tkv + nkv;
   launch_convert_pair(ctx->stream, (const float*)k->ptr, (const float*)v->ptr, (f16*)tkv, nkv);
   rc = run_attention(ctx, a, B);
   pool_release(ctx, tkv, cap);
